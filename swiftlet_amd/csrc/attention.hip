@@ -4,37 +4,42 @@
 // GPU path runs on the host (attnCoreCPU, QwenMetalModel.swift:1086-1134).
 //
 // Two launches, split over the cached positions:
-//   attn_partial  grid (splits, KVH), one wave per query head of the kv
-//                 head's group: the head's query RMS-normalised (q_norm) and
-//                 rotated (partial NeoX RoPE), the new key likewise (k_norm)
-//                 and appended with the new value by the split holding the
-//                 current position; then an online softmax over the split's
-//                 positions: running max m, sum l and sum of p * v.
-//   attn_combine  one wave per query head: the splits merged
+//   attn_partial  grid (splits, KVH): the group's queries RMS-normalised
+//                 (q_norm) and rotated (partial NeoX RoPE), the new key likewise
+//                 (k_norm) and appended with the new value by the split holding
+//                 the current position; then the split's maximum, sum and sum
+//                 of p * v per query head, with an online softmax.
+//   attn_combine  grid (H, blocks of 64 dims): the splits merged
 //                 (exp(m_s - M) weights), divided by the total, times
 //                 sigmoid(gate).
 // The cache is f32 [max_positions][KVH][hd] for k and for v, the order in
 // which the reference appends rows (state.kv).
+#include <algorithm>
 #include <cmath>
 
 #include "internal.hpp"
+#include "route.hpp"
 
 namespace swq {
 namespace {
 
 constexpr int kAttnMaxGroup = 16;  // query heads per kv head
-constexpr int kAttnThreads = 512;
+constexpr int kAttnThreads = 256;
 constexpr int kAttnWaves = kAttnThreads / kWave;
-constexpr int kAttnChunk = 64;     // positions per workgroup (one per lane)
+constexpr int kAttnHeadsPerWave = kAttnMaxGroup / kAttnWaves;
+constexpr int kAttnMaxSplits = 512;
+constexpr int kAttnTargetWgs = 512;
 constexpr int kAttnMaxRot = 256;
 
 struct AttnArgs {
     const float *q_proj, *k_proj, *v_proj;
     const float *q_norm_w, *k_norm_w;
     float *cache_k, *cache_v;
-    float *part;  // [H][splits][hd + 2]
+    float *part;     // [H][splits][hd]: the splits' value sums
+    float *part_ml;  // [H][splits][2]: their maxima and sums
     float *out;   // [H * hd]
-    int32_t H, KVH, hd, rot, group, splits, chunk;
+    int32_t H, KVH, hd, rot, group, splits;
+    int32_t per;  // positions per split
     int32_t position;
     float theta, eps, scale;
     // the rotation of `position`: cos and sin of position * theta^(-2j/rot),
@@ -53,24 +58,50 @@ struct HeadVec {
     float v[EPL];
 };
 
-// RMS-normalise a head vector (x *= scale * w) and rotate its first `rot`
-// elements (pairs j, j + rot/2) with the rotation table, in the reference's
-// operation order.  The wave's copy goes through `lds` (HD floats) so that a
-// lane can read its rotation partner.
+// This lane's elements of the norm weight, and of the rotation table at them:
+// element i < rot turns with its partner i +- rot / 2 by angle i % (rot / 2).
 template <int HD>
-__device__ __forceinline__ void norm_rope(HeadVec<HD> &x, const float *w, float eps, int rot, const float *cs,
-                                          const float *sn, float *lds) {
+struct HeadTable {
+    static constexpr int EPL = HeadVec<HD>::EPL;
+    float w[EPL], c[EPL], s[EPL];
+    __device__ __forceinline__ void load(const float *weight, const AttnArgs &a) {
+        const int lane = threadIdx.x & (kWave - 1), half = a.rot / 2;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            const int i = min(lane * EPL + e, HD - 1);
+            w[e] = weight[i];
+            const int j = i < half ? i : (i < a.rot ? i - half : 0);
+            c[e] = a.rope_cos[j];
+            s[e] = a.rope_sin[j];
+        }
+    }
+};
+
+template <int HD>
+__device__ __forceinline__ void load_head(HeadVec<HD> &x, const float *src) {
+    const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+    for (int e = 0; e < HeadVec<HD>::EPL; ++e)
+        x.v[e] = lane < HeadVec<HD>::LANES ? src[lane * HeadVec<HD>::EPL + e] : 0.f;
+}
+
+// RMS-normalise a head vector (x *= scale * w) and rotate its first `rot`
+// elements (pairs j, j + rot/2), in the reference's operation order.  The
+// wave's copy goes through `lds` (HD floats) so that a lane can read its
+// rotation partner.
+template <int HD>
+__device__ __forceinline__ void norm_rope(HeadVec<HD> &x, const HeadTable<HD> &t, float eps, int rot, float *lds) {
     constexpr int EPL = HeadVec<HD>::EPL, LANES = HeadVec<HD>::LANES;
     const int lane = threadIdx.x & (kWave - 1);
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) ss += x.v[e] * x.v[e];
-    ss = wave_sum(ss);
+    ss = wave_sum_all(ss);
     const float sc = 1.0f / __fsqrt_rn(ss / static_cast<float>(HD) + eps);
     if (lane < LANES) {
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
-            x.v[e] *= sc * w[lane * EPL + e];
+            x.v[e] *= sc * t.w[e];
             lds[lane * EPL + e] = x.v[e];
         }
     }
@@ -82,254 +113,338 @@ __device__ __forceinline__ void norm_rope(HeadVec<HD> &x, const float *w, float 
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
             const int i = lane * EPL + e;
-            if (i < rot) {
-                const int j = i < half ? i : i - half;
-                const float c = cs[j], s = sn[j];
-                const float a = lds[j], b = lds[j + half];
-                x.v[e] = i < half ? a * c - b * s : b * c + a * s;
-            }
+            const float o = lds[i < half ? i + half : (i < rot ? i - half : i)];
+            if (i < rot) x.v[e] = i < half ? x.v[e] * t.c[e] - o * t.s[e] : x.v[e] * t.c[e] + o * t.s[e];
         }
     }
 }
 
-// One workgroup per (64-position chunk, kv head): 8 waves.  The chunk's K
-// and V rows are loaded at the start, K row by row (coalesced), V a dim per
-// thread:
-//   keys    K goes to LDS transposed, [dim][position] (a padded row per dim),
-//           so a lane can walk one position's dims without bank conflicts;
-//   scores  wave w sums dims [w*hd/8, (w+1)*hd/8) of each position (lane)
-//           against each query of the group (broadcast from LDS); the 8
-//           partial sums meet in LDS;
-//   softmax per query head over the chunk (wave-wide max and sum);
-//   values  thread t holds dim t % hd of 64 / (512 / hd) positions and adds
-//           p * v for every head; the position groups meet in LDS.
+// One workgroup of four waves per (split, kv head), a quarter of the head's
+// dims on each wave, walking the split's positions TILES * 16 at a time on the
+// fp32 matrix cores (v_mfma_f32_16x16x4_f32: 32-bit products and sums), K and V
+// straight from global memory to the operands, never through LDS:
+//   scores  A = K: lane (r = lane % 16, q = lane / 16) holds position r's dims
+//           4 KW j + KW q + e (one load of KW floats per j), B = the group's
+//           queries in the same dim order, in registers; the result's lane
+//           (h, q) holds head h's partial scores at positions 4 q + i, i < 4;
+//           the four waves' partials meet in LDS, one barrier per step;
+//   softmax online, a running maximum and sum per head, on every wave alike;
+//   values  A = p: the scores' registers are the operand as they are (k step i
+//           takes positions 4 q + i), B = V: lane (n, q) holds dims VW n + e of
+//           position 4 q + i; the result's lane (n, q) holds heads 4 q + i of
+//           the wave's dims, so no sum crosses waves.
+// Heads past the group are zero queries whose results nothing reads.  The next
+// step's K loads are issued before this one's values, its V loads after them.
+//
+// Bound: at short contexts the chain of launch, first loads, norm and rotation,
+// barrier, two products (~5 us), at long ones the bytes: 33,001 positions read
+// 135 MB in 33 us, 4.1 TB/s.  Before, with scores and values on the VALU over K
+// transposed in LDS (120 KB, one workgroup per CU): 59 us there and 13 us at
+// 4,096 positions, now 8.9.  Measured beside it: 4-wave workgroups with every
+// dim on each wave, 16 positions a wave, sums merged through LDS, 13.3 us at
+// 4,096 and 33 us; four tiles a step (spills), 48 us at 33,001.
 template <int HD>
-__global__ __launch_bounds__(kAttnThreads) void attn_partial(const AttnArgs a) {
+struct AttnDims {
+    static constexpr int DW = HD / kAttnWaves;           // dims per wave
+    static constexpr int KW = DW >= 16 ? 4 : DW / 4;     // floats per K load
+    static constexpr int J = DW / (4 * KW);              // K loads per lane and position
+    static constexpr int VW = DW >= 16 ? DW / 16 : 1;    // floats per V load (lanes past the dims idle)
+};
+
+template <int W>
+__device__ __forceinline__ void load_floats(float (&d)[W], const float *p) {
+    if constexpr (W == 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(p);
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+    } else if constexpr (W == 2) {
+        const float2 v = *reinterpret_cast<const float2 *>(p);
+        d[0] = v.x; d[1] = v.y;
+    } else {
+        d[0] = *p;
+    }
+}
+
+// The maximum that exponents are taken against: 0 where every score so far is -inf, so that
+// such positions count nothing instead of turning the sum into NaN.
+__device__ __forceinline__ float finite_max(float m) { return m == -INFINITY ? 0.f : m; }
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <int HD, int TILES>
+__global__ __launch_bounds__(kAttnThreads, 2) void attn_partial(const AttnArgs a) {
+    using D = AttnDims<HD>;
+    constexpr int DW = D::DW, KW = D::KW, J = D::J, VW = D::VW;
     constexpr int EPL = HeadVec<HD>::EPL;
-    constexpr int DS = HD / kAttnWaves;           // key dims per wave (and K floats per thread)
-    constexpr int VW = HD >= 32 ? 4 : 1;          // K load width
-    constexpr int NK = DS / VW;                   // K loads per thread
-    constexpr int UPR = HD / VW;                  // K load units per row
-    constexpr int PG = kAttnThreads / HD;         // position groups of the value pass
-    constexpr int PPG = kAttnChunk / PG;          // positions per group
-    constexpr int KT = HD * (kAttnChunk + 1);     // transposed K, padded
-    constexpr int AC = PG * kAttnMaxGroup * HD;   // value partials
-    __shared__ float s_q[kAttnMaxGroup][HD];
-    __shared__ float s_knew[HD], s_vnew[HD];
-    __shared__ float s_part[kAttnWaves][kAttnMaxGroup][kAttnChunk + 1];
-    __shared__ float s_e[kAttnMaxGroup][kAttnChunk];
-    __shared__ float s_ml[kAttnMaxGroup][2];
-    __shared__ float s_big[KT > AC ? KT : AC];    // transposed K, later the value partials
+    constexpr int STEP = 16 * TILES;
+    __shared__ __attribute__((aligned(16))) float s_q[kAttnMaxGroup * HD];  // operand order
+    __shared__ __attribute__((aligned(16))) float s_rot[kAttnMaxGroup * HD];
+    __shared__ __attribute__((aligned(16))) float s_new[HD];                // the new key
+    __shared__ f32x4_t s_s[2][kAttnWaves][TILES][kWave];
     const int split = blockIdx.x, g = blockIdx.y;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
-    const int p0 = split * kAttnChunk;
-    const int np = min(kAttnChunk, a.position + 1 - p0);  // positions of this chunk (the last one may be short)
-    const bool has_new = a.position < p0 + kAttnChunk;
-    const int pnew = a.position - p0;                     // the new position within the chunk (if has_new)
+    const int r = lane & 15, q = lane >> 4;
     const int G = a.group;
+    const int64_t row = static_cast<int64_t>(a.KVH) * HD;
+    const int p0 = split * a.per, p1 = min(p0 + a.per, a.position + 1);  // this split's positions: never empty
 
-    // loads first: K unit f = i * 512 + tid is row f / UPR, dims
-    // (f % UPR) * VW ..; V: thread = dim, position group.  Rows past the
-    // chunk or at the new position read nothing (row 0 stands in).
-    float kr[DS], vr[PPG];
+    // this wave's queries (heads wave, wave + 4, ...) and the tables, ahead of K and V
+    HeadVec<HD> qx[kAttnHeadsPerWave];
+    HeadTable<HD> qt;
+    qt.load(a.q_norm_w, a);
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-        const int f = i * kAttnThreads + tid, r = f / UPR, c = (f % UPR) * VW;
-        const bool ok = r < np && r != pnew;
-        const float *src = a.cache_k + (static_cast<int64_t>(ok ? p0 + r : 0) * a.KVH + g) * HD + c;
-        if constexpr (VW == 4) {
-            const float4 v = *reinterpret_cast<const float4 *>(src);
-            kr[4 * i] = ok ? v.x : 0.f;
-            kr[4 * i + 1] = ok ? v.y : 0.f;
-            kr[4 * i + 2] = ok ? v.z : 0.f;
-            kr[4 * i + 3] = ok ? v.w : 0.f;
-        } else {
-            const float v = *src;
-            kr[i] = ok ? v : 0.f;
-        }
-    }
-    const int vd = tid % HD, vg = tid / HD;
+    for (int u = 0; u < kAttnHeadsPerWave; ++u)
+        load_head<HD>(qx[u], a.q_proj + static_cast<int64_t>(g * G + min(u * kAttnWaves + wave, G - 1)) * 2 * HD);
+    // and, on the last wave of the split that holds the new position, its key
+    const bool has_new = wave == kAttnWaves - 1 && a.position < p1;
+    HeadVec<HD> kx, vx;
+    HeadTable<HD> kt = qt;
+    if (has_new) {
+        load_head<HD>(kx, a.k_proj + g * HD);
+        load_head<HD>(vx, a.v_proj + g * HD);
 #pragma unroll
-    for (int j = 0; j < PPG; ++j) {
-        const int pl = vg * PPG + j;
-        const bool ok = pl < np && pl != pnew;
-        const float v = a.cache_v[(static_cast<int64_t>(ok ? p0 + pl : 0) * a.KVH + g) * HD + vd];
-        vr[j] = ok ? v : 0.f;
+        for (int e = 0; e < EPL; ++e) kt.w[e] = a.k_norm_w[min(lane * EPL + e, HD - 1)];
     }
 
-    // the new key and value (wave 0 of the chunk holding the position)
-    if (has_new && wave == 0) {
-        HeadVec<HD> k;
+    float kr[TILES][J][KW], vr[TILES][4][VW];
+    const float *ck = a.cache_k + g * HD + wave * DW + KW * q;
+    const float *cv = a.cache_v + g * HD + wave * DW + min(VW * r, DW - VW);
+    // K and V of the step at t0; rows past the split's positions read its last one
+    auto load_k = [&](int t0) {
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) k.v[e] = 0.f;
-        if (lane < HeadVec<HD>::LANES) {
+        for (int t = 0; t < TILES; ++t) {
+            const float *p = ck + min(t0 + 16 * t + r, p1 - 1) * row;
 #pragma unroll
-            for (int e = 0; e < EPL; ++e) k.v[e] = a.k_proj[g * HD + lane * EPL + e];
+            for (int j = 0; j < J; ++j) load_floats<KW>(kr[t][j], p + 4 * KW * j);
         }
-        norm_rope<HD>(k, a.k_norm_w, a.eps, a.rot, a.rope_cos, a.rope_sin, s_q[0]);
+    };
+    auto load_v = [&](int t0) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_floats<VW>(vr[t][i], cv + min(t0 + 16 * t + 4 * q + i, p1 - 1) * row);
+    };
+    load_k(p0);
+    load_v(p0);
+
+    // the new position's key and value: into the cache, the key into LDS too
+    if (has_new) {
+        norm_rope<HD>(kx, kt, a.eps, a.rot, s_new);
+        __builtin_amdgcn_wave_barrier();
+        const int64_t at = a.position * row + g * HD;
         if (lane < HeadVec<HD>::LANES) {
-            float *ck = a.cache_k + (static_cast<int64_t>(a.position) * a.KVH + g) * HD;
-            float *cv = a.cache_v + (static_cast<int64_t>(a.position) * a.KVH + g) * HD;
 #pragma unroll
             for (int e = 0; e < EPL; ++e) {
                 const int i = lane * EPL + e;
-                const float vv = a.v_proj[g * HD + i];
-                s_knew[i] = k.v[e];
-                s_vnew[i] = vv;
-                ck[i] = k.v[e];
-                cv[i] = vv;
+                s_new[i] = kx.v[e];
+                a.cache_k[at + i] = kx.v[e];
+                a.cache_v[at + i] = vx.v[e];
+            }
+        }
+    }
+    // the group's queries, into operand order: element i of head h at lane
+    // (h, q), load j of its wave; zeros for the heads past the group
+#pragma unroll
+    for (int u = 0; u < kAttnHeadsPerWave; ++u) {
+        const int hh = u * kAttnWaves + wave;
+        if (hh < G) norm_rope<HD>(qx[u], qt, a.eps, a.rot, s_rot + hh * HD);
+        if (lane < HeadVec<HD>::LANES) {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                const int i = lane * EPL + e;
+                s_q[((i / (4 * KW)) * kWave + ((i / KW) & 3) * 16 + hh) * KW + i % KW] = hh < G ? qx[u].v[e] : 0.f;
             }
         }
     }
     lds_barrier();
-    // the group's queries, normalised and rotated, into LDS
-    for (int hh = wave; hh < G; hh += kAttnWaves) {
-        const int h = g * G + hh;
-        HeadVec<HD> q;
+    float qf[J][KW];
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) q.v[e] = 0.f;
-        if (lane < HeadVec<HD>::LANES) {
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) q.v[e] = a.q_proj[static_cast<int64_t>(h) * 2 * HD + lane * EPL + e];
-        }
-        norm_rope<HD>(q, a.q_norm_w, a.eps, a.rot, a.rope_cos, a.rope_sin, s_q[hh]);
-        __builtin_amdgcn_wave_barrier();
-        if (lane < HeadVec<HD>::LANES) {
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) s_q[hh][lane * EPL + e] = q.v[e];
-        }
-    }
-    // K into LDS, transposed; the new row from its LDS copy
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-        const int f = i * kAttnThreads + tid, r = f / UPR, c = (f % UPR) * VW;
-#pragma unroll
-        for (int e = 0; e < VW; ++e) {
-            const float v = (has_new && r == pnew) ? s_knew[c + e] : kr[VW * i + e];
-            s_big[(c + e) * (kAttnChunk + 1) + r] = v;
-        }
-    }
-    if (has_new) {
-#pragma unroll
-        for (int j = 0; j < PPG; ++j)
-            if (vg * PPG + j == pnew) vr[j] = s_vnew[vd];
-    }
-    lds_barrier();
+    for (int j = 0; j < J; ++j) load_floats<KW>(qf[j], &s_q[((wave * J + j) * kWave + lane) * KW]);
 
-    // scores: partial dots over this wave's dims (lane = position)
-    for (int hh = 0; hh < G; ++hh) {
-        float d = 0.f;
+    float m = -INFINITY, l = 0.f;  // of head r (m the same in its four q lanes, l this lane's share)
+    f32x4_t acc[VW];
 #pragma unroll
-        for (int i = 0; i < DS; ++i) d += s_big[(wave * DS + i) * (kAttnChunk + 1) + lane] * s_q[hh][wave * DS + i];
-        s_part[wave][hh][lane] = d;
+    for (int e = 0; e < VW; ++e) acc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    int par = 0;
+    for (int t0 = p0; t0 < p1; t0 += STEP, par ^= 1) {
+        const int pn = a.position - t0;  // the new row within the step, if 0 <= pn < STEP
+        if (pn < STEP) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+                if (16 * t + r == pn) {
+#pragma unroll
+                    for (int j = 0; j < J; ++j) load_floats<KW>(kr[t][j], &s_new[wave * DW + 4 * KW * j + KW * q]);
+                }
+        }
+        f32x4_t sc[TILES], sc2[TILES];  // two chains per tile
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) sc[t] = sc2[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int e = 0; e < KW; ++e)
+#pragma unroll
+                for (int t = 0; t < TILES; ++t) {
+                    f32x4_t &c = (e & 1) ? sc2[t] : sc[t];
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t][j][e], qf[j][e], c, 0, 0, 0);
+                }
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) s_s[par][wave][t][lane] = sc[t] + sc2[t];
+        if (t0 + STEP < p1) load_k(t0 + STEP);
+        lds_barrier();
+        float p[TILES][4], mt = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const f32x4_t x = (s_s[par][0][t][lane] + s_s[par][1][t][lane]) + (s_s[par][2][t][lane] + s_s[par][3][t][lane]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[t][i] = t0 + 16 * t + 4 * q + i < p1 ? x[i] * a.scale : -INFINITY;
+                mt = fmaxf(mt, p[t][i]);
+            }
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, kWave));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
+        const float mn = fmaxf(m, mt);
+        const float ref = finite_max(mn);
+        const float alpha = expf(m - ref);  // 0 for the first step
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                p[t][i] = expf(p[t][i] - ref);
+                l += p[t][i];
+            }
+        if (t0 != p0) {
+            f32x4_t f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) f[i] = __shfl(alpha, 4 * q + i, kWave);
+#pragma unroll
+            for (int e = 0; e < VW; ++e) acc[e] *= f;
+        }
+        if (t0 + STEP > p1 - (a.position < p1)) {
+            // rows past the end count nothing, whatever they hold; the new row is the projection's
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int at = 16 * t + 4 * q + i;
+                    if (t0 + at >= p1) {
+#pragma unroll
+                        for (int e = 0; e < VW; ++e) vr[t][i][e] = 0.f;
+                    } else if (at == pn) {
+#pragma unroll
+                        for (int e = 0; e < VW; ++e) vr[t][i][e] = a.v_proj[g * HD + wave * DW + min(VW * r, DW - VW) + e];
+                    }
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < VW; ++e)
+                    acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t][i], vr[t][i][e], acc[e], 0, 0, 0);
+        if (t0 + STEP < p1) load_v(t0 + STEP);
     }
-    lds_barrier();
-    // softmax per head over the chunk: wave w takes heads w, w + 8
-    for (int hh = wave; hh < G; hh += kAttnWaves) {
-        float sc = 0.f;
+    l += __shfl_xor(l, 16, kWave);
+    l += __shfl_xor(l, 32, kWave);
+    if (VW * r < DW) {
 #pragma unroll
-        for (int w = 0; w < kAttnWaves; ++w) sc += s_part[w][hh][lane];
-        sc = lane < np ? sc * a.scale : -INFINITY;
-        const float m = wave_max(sc);
-        const float e = lane < np ? expf(sc - m) : 0.f;
-        const float l = wave_sum(e);
-        s_e[hh][lane] = e;
-        if (lane == 0) {
-            s_ml[hh][0] = m;
-            s_ml[hh][1] = l;
+        for (int i = 0; i < 4; ++i) {
+            if (4 * q + i < G) {
+                float *dst = a.part + (static_cast<int64_t>(g * G + 4 * q + i) * a.splits + split) * HD + wave * DW + VW * r;
+#pragma unroll
+                for (int e = 0; e < VW; ++e) dst[e] = acc[e][i];
+            }
         }
     }
-    lds_barrier();
-    // values: p * v for every head (the value partials reuse the K space)
-    float *s_acc = s_big;
-    for (int hh = 0; hh < G; ++hh) {
-        float acc = 0.f;
-#pragma unroll
-        for (int j = 0; j < PPG; ++j) acc += s_e[hh][vg * PPG + j] * vr[j];
-        s_acc[(vg * kAttnMaxGroup + hh) * HD + vd] = acc;
-    }
-    lds_barrier();
-    for (int t = tid; t < G * HD; t += kAttnThreads) {
-        const int hh = t / HD, d = t % HD;
-        float acc = 0.f;
-#pragma unroll
-        for (int q = 0; q < PG; ++q) acc += s_acc[(q * kAttnMaxGroup + hh) * HD + d];
-        a.part[(static_cast<int64_t>(g * G + hh) * a.splits + split) * (HD + 2) + d] = acc;
-    }
-    if (tid < G) {
-        float *dst = a.part + (static_cast<int64_t>(g * G + tid) * a.splits + split) * (HD + 2);
-        dst[HD] = s_ml[tid][0];
-        dst[HD + 1] = s_ml[tid][1];
+    if (tid < G) {  // wave 0, lane (h, 0)
+        float *dst = a.part_ml + (static_cast<int64_t>(g * G + tid) * a.splits + split) * 2;
+        dst[0] = m;
+        dst[1] = l;
     }
 }
 
-// One workgroup of 1024 threads per query head: the splits' maxima and
-// weighted sums reduced across the threads (M = max m_s, L = sum
-// exp(m_s - M) l_s), then thread (d, q) sums exp(m_s - M) * acc_s[d] over
-// every SG-th split (SG = 1024 / hd), four splits per round; the SG partial
-// sums meet in LDS; out = acc / L * sigmoid(gate).
-constexpr int kCombineThreads = 1024;
-
-__device__ __forceinline__ float block_reduce(float v, float *s_red, bool is_max) {
-    v = is_max ? wave_max(v) : wave_sum(v);
-    __syncthreads();
-    if ((threadIdx.x & (kWave - 1)) == 0) s_red[threadIdx.x / kWave] = v;
-    __syncthreads();
-    float r = s_red[0];
-    for (int i = 1; i < kCombineThreads / kWave; ++i) r = is_max ? fmaxf(r, s_red[i]) : r + s_red[i];
-    return r;
-}
+// The splits merged: one workgroup of 512 threads per (query head, 64 dims).
+// M = max m_s and L = sum exp(m_s - M) l_s over the threads (a split each),
+// the weights exp(m_s - M) to LDS; 16 lanes read a split's 64 dims, so a wave
+// takes four splits and the workgroup 32 per round, the first rounds' loads
+// issued before the weights are known; the sums meet over the lanes and in
+// LDS; out = sum / L * sigmoid(gate).  Bound: launch and two round trips, 3.9
+// us at 256 splits (one workgroup per head took 5.2 us at 64 splits, 22 at 516).
+constexpr int kCombineThreads = 512;
+constexpr int kCombineWaves = kCombineThreads / kWave;
+static_assert(kAttnMaxSplits <= kCombineThreads, "a thread per split");
 
 template <int HD>
 __global__ __launch_bounds__(kCombineThreads) void attn_combine(const AttnArgs a) {
-    constexpr int SG = kCombineThreads / HD;
-    constexpr int U = 8;  // splits per round of a thread's value loop
-    __shared__ float s_red[kCombineThreads / kWave];
-    __shared__ float s_acc[SG][HD];
-    const int h = blockIdx.x, tid = threadIdx.x;
-    const int64_t stride = HD + 2;
-    const float *src = a.part + static_cast<int64_t>(h) * a.splits * stride;
-    // maxima and sums: one load round per 1024 splits
-    float m = -INFINITY, mm[4], ll[4];
-    int n = 0;
-    for (int s = tid; s < a.splits; s += kCombineThreads, ++n) {
-        if (n < 4) {
-            mm[n] = src[s * stride + HD];
-            ll[n] = src[s * stride + HD + 1];
-            m = fmaxf(m, mm[n]);
-        } else {
-            m = fmaxf(m, src[s * stride + HD]);
-        }
-    }
-    const float M = block_reduce(m, s_red, true);
-    float l = 0.f;
-    n = 0;
-    for (int s = tid; s < a.splits; s += kCombineThreads, ++n)
-        l += n < 4 ? expf(mm[n] - M) * ll[n] : expf(src[s * stride + HD] - M) * src[s * stride + HD + 1];
-    const float L = block_reduce(l, s_red, false);
-    // values: thread (d, q) takes splits q, q + SG, ..., U per round
-    const int d = tid % HD, q = tid / HD;
-    float acc = 0.f;
-    int s = q;
-    for (; s + (U - 1) * SG < a.splits; s += U * SG) {
-        float w[U], v[U];
+    constexpr int DB = HD < 64 ? HD : 64;           // dims per workgroup
+    constexpr int LPS = DB / 4;                     // lanes per split (4 dims each)
+    constexpr int SPR = kCombineThreads / LPS;      // splits per round
+    constexpr int U = 8;                            // rounds in flight
+    __shared__ float s_w[kAttnMaxSplits];
+    __shared__ float s_red[2][kCombineWaves];
+    __shared__ float s_acc[kCombineWaves][DB];
+    const int h = blockIdx.x, d0 = blockIdx.y * DB, tid = threadIdx.x;
+    const int wave = tid / kWave, lane = tid & (kWave - 1);
+    const float *ml = a.part_ml + static_cast<int64_t>(h) * a.splits * 2;
+    const float *src = a.part + static_cast<int64_t>(h) * a.splits * HD + d0 + (tid % LPS) * 4;
+    const int s0 = tid / LPS;
+    const bool mine = tid < a.splits;
+    const float ms = mine ? ml[2 * tid] : -INFINITY;
+    const float ls = mine ? ml[2 * tid + 1] : 0.f;
+    const float gate = a.q_proj[static_cast<int64_t>(h) * 2 * HD + HD + d0 + tid % DB];
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        v[u] = *reinterpret_cast<const float4 *>(src + static_cast<int64_t>(min(s0 + u * SPR, a.splits - 1)) * HD);
+    float M = wave_max(ms);
+    if (lane == 0) s_red[0][wave] = M;
+    lds_barrier();
+#pragma unroll
+    for (int w = 0; w < kCombineWaves; ++w) M = fmaxf(M, s_red[0][w]);
+    const float wt = mine ? expf(ms - finite_max(M)) : 0.f;
+    if (tid < a.splits) s_w[tid] = wt;
+    const float lw = wave_sum(wt * ls);
+    if (lane == 0) s_red[1][wave] = lw;
+    lds_barrier();
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int base = 0; base < a.splits; base += U * SPR) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            w[u] = src[(s + u * SG) * stride + HD];
-            v[u] = src[(s + u * SG) * stride + d];
+            const int s = base + s0 + u * SPR;
+            if (s < a.splits) {
+                const float w = s_w[s];
+                acc[0] += w * v[u].x;
+                acc[1] += w * v[u].y;
+                acc[2] += w * v[u].z;
+                acc[3] += w * v[u].w;
+            }
         }
+        if (base + U * SPR < a.splits) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc += expf(w[u] - M) * v[u];
+            for (int u = 0; u < U; ++u)
+                v[u] = *reinterpret_cast<const float4 *>(
+                    src + static_cast<int64_t>(min(base + (U + u) * SPR + s0, a.splits - 1)) * HD);
+        }
     }
-    for (; s < a.splits; s += SG) acc += expf(src[s * stride + HD] - M) * src[s * stride + d];
-    s_acc[q][d] = acc;
-    __syncthreads();
-    if (tid < HD) {
-        float t = 0.f;
 #pragma unroll
-        for (int i = 0; i < SG; ++i) t += s_acc[i][tid];
-        const float gate = a.q_proj[static_cast<int64_t>(h) * 2 * HD + HD + tid];
-        a.out[h * HD + tid] = (t / L) * sigmoid_acc(gate);
+    for (int e = 0; e < 4; ++e) {
+        for (int off = LPS; off < kWave; off <<= 1) acc[e] += __shfl_xor(acc[e], off, kWave);
+    }
+    if (lane < LPS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s_acc[wave][lane * 4 + e] = acc[e];
+    }
+    lds_barrier();
+    if (tid < DB) {
+        float L = 0.f, t = 0.f;
+#pragma unroll
+        for (int w = 0; w < kCombineWaves; ++w) L += s_red[1][w];
+#pragma unroll
+        for (int w = 0; w < kCombineWaves; ++w) t += s_acc[w][tid];
+        a.out[h * HD + d0 + tid] = (t / L) * sigmoid_acc(gate);
     }
 }
 
@@ -352,10 +467,32 @@ size_t half_cache(const swq_attention_layer *l) {
     return align256(static_cast<size_t>(l->max_positions) * l->num_kv_heads * l->head_dim * sizeof(float));
 }
 
+// The split of n positions over workgroups: one 16-position tile a workgroup while that takes
+// no more than two workgroups per CU over all kv heads (a CU's loads come in at about 32 KB per
+// round trip, so a short context is fastest spread thin), else that many workgroups, each
+// walking its positions two tiles a step.  Step + merge at 33,001 positions and 2 kv heads:
+// 256 workgroups 42.7 us, 512 38.5, 1,024 41.0; at 4,096 13.5, 13.7, 13.6; at 1,000 the
+// 64-position workgroups of four waves took 15.0, one tile each 10.2.
+struct AttnPlan {
+    int per, splits, tiles;
+};
+
+int64_t split_cap(int kvh) { return std::min(kAttnMaxSplits, std::max(1, kAttnTargetWgs / kvh)); }
+
+AttnPlan plan_splits(int64_t n, int kvh) {
+    const int64_t cap = split_cap(kvh), per = std::max<int64_t>((n + cap - 1) / cap, 16);
+    return {static_cast<int>(per), static_cast<int>((n + per - 1) / per), per <= 16 ? 1 : 2};
+}
+
+// Most splits of any length up to n.
+int64_t most_splits(int64_t n, int kvh) { return std::min<int64_t>((n + 15) / 16, split_cap(kvh)); }
+
 template <int HD>
-void launch(const AttnArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL(attn_partial<HD>, dim3(a.splits, a.KVH), dim3(kAttnThreads), 0, s, a);
-    hipLaunchKernelGGL(attn_combine<HD>, dim3(a.H), dim3(kCombineThreads), 0, s, a);
+void launch(const AttnArgs &a, int tiles, hipStream_t s) {
+    const dim3 grid(a.splits, a.KVH), block(kAttnThreads);
+    if (tiles == 1) hipLaunchKernelGGL((attn_partial<HD, 1>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((attn_partial<HD, 2>), grid, block, 0, s, a);
+    hipLaunchKernelGGL(attn_combine<HD>, dim3(a.H, HD < 64 ? 1 : HD / 64), dim3(kCombineThreads), 0, s, a);
 }
 
 }  // namespace
@@ -369,7 +506,7 @@ extern "C" size_t swq_attention_cache_bytes(const swq_attention_layer *l) {
 
 extern "C" size_t swq_attention_workspace_bytes(const swq_attention_layer *l) {
     if (check_layer(l) != SWQ_OK) return 0;
-    const size_t splits = (static_cast<size_t>(l->max_positions) + kAttnChunk - 1) / kAttnChunk;
+    const size_t splits = most_splits(l->max_positions, l->num_kv_heads);
     return static_cast<size_t>(l->num_heads) * splits * (l->head_dim + 2) * sizeof(float);
 }
 
@@ -400,8 +537,10 @@ extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_p
     a.rot = l->rotary_dims;
     a.group = a.H / a.KVH;
     a.position = static_cast<int32_t>(position);
-    a.chunk = kAttnChunk;
-    a.splits = (a.position + kAttnChunk) / kAttnChunk;  // chunks holding positions 0..position
+    const AttnPlan plan = plan_splits(position + 1, a.KVH);
+    a.per = plan.per;
+    a.splits = plan.splits;
+    a.part_ml = a.part + static_cast<int64_t>(a.H) * a.splits * a.hd;
     a.theta = l->rope_theta;
     a.eps = l->norm_eps;
     // the rotation table: powf / cosf / sinf of the reference's float
@@ -417,11 +556,11 @@ extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_p
     a.scale = 1.0f / std::sqrt(static_cast<float>(a.hd));
     hipStream_t s = static_cast<hipStream_t>(stream);
     switch (a.hd) {
-        case 16: launch<16>(a, s); break;
-        case 32: launch<32>(a, s); break;
-        case 64: launch<64>(a, s); break;
-        case 128: launch<128>(a, s); break;
-        default: launch<256>(a, s); break;
+        case 16: launch<16>(a, plan.tiles, s); break;
+        case 32: launch<32>(a, plan.tiles, s); break;
+        case 64: launch<64>(a, plan.tiles, s); break;
+        case 128: launch<128>(a, plan.tiles, s); break;
+        default: launch<256>(a, plan.tiles, s); break;
     }
     return launch_status();
 }

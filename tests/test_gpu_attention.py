@@ -105,6 +105,43 @@ def test_real_shape_long_cache(position):
     assert err < 1e-5
 
 
+@pytest.mark.parametrize("H,KVH,hd,rot,position", [
+    (1, 1, 16, 4, 0), (16, 1, 16, 16, 15), (6, 2, 32, 8, 16), (3, 3, 64, 0, 17), (16, 1, 128, 32, 31),
+    (16, 2, 256, 64, 32), (16, 2, 256, 2, 4094), (16, 2, 256, 2, 4095), (16, 2, 256, 2, 4096), (5, 1, 64, 2, 8191),
+    (16, 2, 256, 2, 8191), (16, 2, 256, 2, 8192), (16, 8, 128, 2, 2113)])
+def test_split_edges(H, KVH, hd, rot, position):
+    """Positions at the edges of a 16-position tile, of a split of one tile (512 / KVH of them,
+    at most 512) and of a step of two tiles; every head size, groups of 1 to 16.  Rows of the
+    cache past the position hold NaN, as does the new row before the step.  From position 2,000
+    on two dims rotate: their angle is the position itself, while theta^(-2j/rot), j > 0, may
+    differ in its last bit from NumPy's float32 power, which moves the angle by up to position *
+    2^-24 (2e-4 at 4,094), in any order of the sums.  Bar: that of the
+    other cases, 1e-5 of the largest output (sums of up to 8,193 fp32 products in blocks:
+    ~2^-24 * sqrt(8193) = 5e-6)."""
+    import torch
+    rng = np.random.default_rng(1000 * H + position)
+    prm = dict(q_norm_w=(1 + 0.2 * rng.standard_normal(hd)).astype(f32), k_norm_w=(1 + 0.2 * rng.standard_normal(hd)).astype(f32),
+               H=H, KVH=KVH, hd=hd, rot=rot, theta=1e7, eps=1e-6)
+    blk = _block(prm, position + 40)
+    cache, ws = blk.new_cache(), blk.new_workspace()
+    gk, gv = blk.cache_views(cache)
+    ck = (rng.standard_normal((position, KVH, hd)) * 0.5).astype(f32)
+    cv = rng.standard_normal((position, KVH, hd)).astype(f32)
+    gk[position:].fill_(float("nan"))
+    gv[position:].fill_(float("nan"))
+    gk[:position].copy_(torch.from_numpy(ck))
+    gv[:position].copy_(torch.from_numpy(cv))
+    q, k, v = (rng.standard_normal((1, n)).astype(f32) for n in (H * 2 * hd, KVH * hd, KVH * hd))
+    want, wk, wv = A.attention_core(q, k, v, cache_k=ck, cache_v=cv, **prm)
+    print(f"H {H} KVH {KVH} hd {hd} position {position}", flush=True)
+    out = blk.step(*(torch.from_numpy(t[0]).cuda() for t in (q, k, v)), cache, ws, position)
+    torch.cuda.synchronize()
+    assert _rel(out.cpu().numpy(), want[0]) < 1e-5
+    assert _rel(gk[position].cpu().numpy(), wk[-1]) < 1e-5
+    assert np.array_equal(gv[position].cpu().numpy(), wv[-1])
+    assert torch.isnan(gk[position + 1:]).all() and np.array_equal(gk[:position].cpu().numpy(), ck)
+
+
 def test_tiny_q4_model_entirely_on_the_device_matches_mlx():
     import torch
     from safetensors.numpy import load_file
