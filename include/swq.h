@@ -208,8 +208,8 @@ size_t swq_sample_workspace_bytes(int vocab);
  * to the lower id), p_i = exp((l_i - l_0) / temperature), the top-p cut and
  * the draw r = u * sum p, the first i with r - (p_0 + .. + p_i) <= 0.
  * u in [0, 1) is the caller's uniform number (the reference draws
- * Float.random).  out_token: one int32 on the device.  Id lists and counts
- * are device arrays.  Replaces SwiftletSession.sample
+ * Float.random).  out_token: one int32 that the device can write (its own or
+ * pinned host memory).  Id lists and counts are device arrays.  Replaces SwiftletSession.sample
  * (SwiftletSession.swift:226-273). */
 int swq_sample(const float *logits, int vocab, const swq_sample_options *options,
                const int32_t *seen_ids, const int32_t *seen_counts, int n_seen,
@@ -264,6 +264,17 @@ size_t swq_deltanet_state_bytes(const swq_deltanet_layer *layer);
 int swq_deltanet_step(const swq_deltanet_layer *layer, const float *qkvz, const float *ba, void *state,
                       size_t state_bytes, int64_t position, float *out, void *stream);
 
+/* The whole block for one token in one call: the projections of x (one launch;
+ * with norm_weight, x is the un-normalised hidden state), swq_deltanet_step and
+ * out_proj (f32 out).  projections: SPLIT qkv, z, b, a; INTERLEAVED qkvz, ba.
+ * scratch: swq_deltanet_scratch_floats(layer) f32 device words, 16-byte
+ * aligned, dead after the call's work. */
+size_t swq_deltanet_scratch_floats(const swq_deltanet_layer *layer);
+int swq_deltanet_token(const swq_deltanet_layer *layer, const swq_qlinear *projections, int n_projections,
+                       const swq_qlinear *out_proj, const float *x, const void *norm_weight, int norm_dtype,
+                       float norm_eps, void *state, size_t state_bytes, int64_t position, float *scratch,
+                       size_t scratch_floats, float *out, void *stream);
+
 /* ---- gated GQA attention decode step ------------------------------------ */
 
 /* One full-attention block (self_attn) between q/k/v_proj and o_proj. */
@@ -302,6 +313,17 @@ size_t swq_attention_workspace_bytes(const swq_attention_layer *layer);
 int swq_attention_step(const swq_attention_layer *layer, const float *q_proj, const float *k_proj,
                        const float *v_proj, void *cache, size_t cache_bytes, int64_t position, float *out,
                        void *ws, size_t ws_bytes, void *stream);
+
+/* The whole block for one token in one call: q/k/v_proj of x (one launch; with
+ * norm_weight, x is the un-normalised hidden state), swq_attention_step and
+ * o_proj (f32 out).  projections: q, k, v, of at least 2*H*hd, KVH*hd and
+ * KVH*hd rows.  scratch: swq_attention_scratch_floats f32 device words, 16-byte
+ * aligned, dead after the call's work. */
+size_t swq_attention_scratch_floats(const swq_attention_layer *layer, const swq_qlinear *projections);
+int swq_attention_token(const swq_attention_layer *layer, const swq_qlinear *projections,
+                        const swq_qlinear *o_proj, const float *x, const void *norm_weight, int norm_dtype,
+                        float norm_eps, void *cache, size_t cache_bytes, int64_t position, float *scratch,
+                        size_t scratch_floats, float *out, void *ws, size_t ws_bytes, void *stream);
 
 /* ---- checkpoint and .qpack loading ----------------------------------- */
 

@@ -131,6 +131,12 @@ SIGNATURES = {
     "swq_attention_cache_bytes": (_SZ, [_c.POINTER(AttentionLayer)]),
     "swq_attention_workspace_bytes": (_SZ, [_c.POINTER(AttentionLayer)]),
     "swq_attention_step": (_I, [_c.POINTER(AttentionLayer), _P, _P, _P, _P, _SZ, _I64, _P, _P, _SZ, _P]),
+    "swq_deltanet_scratch_floats": (_SZ, [_c.POINTER(DeltaNetLayer)]),
+    "swq_deltanet_token": (_I, [_c.POINTER(DeltaNetLayer), _c.POINTER(QLinear), _I, _c.POINTER(QLinear), _P, _P, _I,
+                                _c.c_float, _P, _SZ, _I64, _P, _SZ, _P, _P]),
+    "swq_attention_scratch_floats": (_SZ, [_c.POINTER(AttentionLayer), _c.POINTER(QLinear)]),
+    "swq_attention_token": (_I, [_c.POINTER(AttentionLayer), _c.POINTER(QLinear), _c.POINTER(QLinear), _P, _P, _I,
+                                 _c.c_float, _P, _SZ, _I64, _P, _SZ, _P, _P, _SZ, _P]),
     "swq_checkpoint_open": (_I, [_c.c_char_p, _c.POINTER(_P)]),
     "swq_checkpoint_close": (None, [_P]),
     "swq_checkpoint_tensor_count": (_I, [_P]),

@@ -11,7 +11,7 @@ import ctypes
 
 from . import _lib
 from ._lib import AttentionLayer, check
-from .engine import GPULinear, HipEngine, _stream_handle, _torch
+from .engine import DescArray, GPULinear, HipEngine, _norm_arg, _stream_handle, _torch
 
 
 class AttentionGPU:
@@ -34,6 +34,7 @@ class AttentionGPU:
                                  rotary_dims=rotary_dims, rope_theta=rope_theta, norm_eps=eps,
                                  max_positions=max_positions, reserved=0, q_norm_weight=self.q_norm.data_ptr(),
                                  k_norm_weight=self.k_norm.data_ptr())
+        self._projs = DescArray()
 
     def _bytes(self, fn, what):
         n = fn(ctypes.byref(self._c))
@@ -76,15 +77,17 @@ class AttentionGPU:
         """x [H_model] f32 -> the block's output: q/k/v_proj in one launch
         (with norm_weight, x is the un-normalised hidden state and the input
         RMSNorm runs inside that launch), the step, o_proj."""
-        torch = _torch()
+        empty, f32, dev = _torch().empty, _torch().float32, x.device
         pq, pk, pv = self.projections
-        q = torch.empty(pq.out_dim, dtype=torch.float32, device=x.device)
-        k = torch.empty(pk.out_dim, dtype=torch.float32, device=x.device)
-        v = torch.empty(pv.out_dim, dtype=torch.float32, device=x.device)
-        engine.encode_gemv_multi([pq, pk, pv], x, [q, k, v], norm_weight=norm_weight, eps=eps, stream=stream)
-        att = self.step(q, k, v, cache, ws, position, stream=stream)
-        r = torch.empty(self.o_proj.out_dim, dtype=torch.float32, device=x.device)
-        engine.encode_gemv(self.o_proj, att, r, stream=stream)
+        projs = self._projs.of((pq, pk, pv))
+        n = self.lib.swq_attention_scratch_floats(ctypes.byref(self._c), projs)
+        scratch = empty(n, dtype=f32, device=dev)
+        r = empty(self.o_proj.out_dim, dtype=f32, device=dev)
+        wdt, wptr = _norm_arg(norm_weight)
+        check(self.lib.swq_attention_token(
+            ctypes.byref(self._c), projs, self.o_proj.desc(), x.data_ptr(), wptr, wdt, eps, cache.data_ptr(),
+            cache.numel(), position, scratch.data_ptr(), n, r.data_ptr(), ws.data_ptr(), ws.numel(),
+            _stream_handle(stream)), "attention_token")
         return r
 
 

@@ -564,3 +564,32 @@ extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_p
     }
     return launch_status();
 }
+
+// The block's four launches from one entry, as swq_deltanet_token.
+extern "C" size_t swq_attention_scratch_floats(const swq_attention_layer *l, const swq_qlinear *projections) {
+    if (check_layer(l) != SWQ_OK || !projections) return 0;
+    int64_t n = 1LL * l->num_heads * l->head_dim;
+    for (int i = 0; i < 3; ++i) n += pad_floats(std::max(projections[i].out_dim, 0));
+    return static_cast<size_t>(n);
+}
+
+extern "C" int swq_attention_token(const swq_attention_layer *l, const swq_qlinear *projections,
+                                   const swq_qlinear *o_proj, const float *x, const void *norm_weight, int norm_dtype,
+                                   float norm_eps, void *cache, size_t cache_bytes, int64_t position, float *scratch,
+                                   size_t scratch_floats, float *out, void *ws, size_t ws_bytes, void *stream) {
+    int st = check_layer(l);
+    if (st != SWQ_OK) return st;
+    if (!projections || !o_proj || !scratch || !out) return SWQ_ERR_INVALID_ARGUMENT;
+    const int64_t val = 1LL * l->num_heads * l->head_dim, kv = 1LL * l->num_kv_heads * l->head_dim;
+    if (projections[0].out_dim < 2 * val || projections[1].out_dim < kv || projections[2].out_dim < kv ||
+        o_proj->in_dim > val)
+        return SWQ_ERR_BAD_SHAPE;
+    if (scratch_floats < swq_attention_scratch_floats(l, projections)) return SWQ_ERR_WORKSPACE;
+    float *q = scratch, *k = q + pad_floats(projections[0].out_dim), *v = k + pad_floats(projections[1].out_dim);
+    float *y = v + pad_floats(projections[2].out_dim);
+    float *ys[3] = {q, k, v};
+    st = swq_encode_gemv_multi(projections, 3, ys, x, norm_weight, norm_dtype, norm_eps, stream);
+    if (st == SWQ_OK) st = swq_attention_step(l, q, k, v, cache, cache_bytes, position, y, ws, ws_bytes, stream);
+    if (st == SWQ_OK) st = swq_encode_gemv(o_proj, 0, 0, 0, 0, y, 0, out, 0, stream);
+    return st;
+}

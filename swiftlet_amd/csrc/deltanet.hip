@@ -295,3 +295,37 @@ extern "C" int swq_deltanet_step(const swq_deltanet_layer *l, const float *qkvz,
     }
     return launch_status();
 }
+
+// The block's three launches from one entry: a caller in another language pays one crossing
+// instead of three (with the descriptors rebuilt for each, a token's block took ~40 us of host
+// time through ctypes, twice the device's 21 us).
+extern "C" size_t swq_deltanet_scratch_floats(const swq_deltanet_layer *l) {
+    if (check_layer(l) != SWQ_OK) return 0;
+    const int64_t val = 1LL * l->num_value_heads * l->value_head_dim;
+    const int64_t qkvz = 2LL * l->num_key_heads * l->key_head_dim + 2 * val;
+    return static_cast<size_t>(pad_floats(qkvz) + pad_floats(2LL * l->num_value_heads) + val);
+}
+
+extern "C" int swq_deltanet_token(const swq_deltanet_layer *l, const swq_qlinear *projections, int n_projections,
+                                  const swq_qlinear *out_proj, const float *x, const void *norm_weight,
+                                  int norm_dtype, float norm_eps, void *state, size_t state_bytes, int64_t position,
+                                  float *scratch, size_t scratch_floats, float *out, void *stream) {
+    int st = check_layer(l);
+    if (st != SWQ_OK) return st;
+    if (!projections || !out_proj || !scratch || !out) return SWQ_ERR_INVALID_ARGUMENT;
+    const int64_t nv = l->num_value_heads, val = nv * l->value_head_dim;
+    const int64_t conv = 2LL * l->num_key_heads * l->key_head_dim + val;
+    if (scratch_floats < swq_deltanet_scratch_floats(l)) return SWQ_ERR_WORKSPACE;
+    float *qkvz = scratch, *ba = qkvz + pad_floats(conv + val), *y = ba + pad_floats(2 * nv);
+    const bool split = l->layout == SWQ_DELTA_SPLIT;
+    float *ys[4] = {qkvz, split ? qkvz + conv : ba, ba, ba + nv};
+    const int64_t rows_split[4] = {conv, val, nv, nv}, rows_fused[2] = {conv + val, 2 * nv};
+    if (n_projections != (split ? 4 : 2)) return SWQ_ERR_BAD_SHAPE;
+    for (int i = 0; i < n_projections; ++i)
+        if (projections[i].out_dim > (split ? rows_split : rows_fused)[i]) return SWQ_ERR_BAD_SHAPE;
+    if (out_proj->in_dim > val) return SWQ_ERR_BAD_SHAPE;
+    st = swq_encode_gemv_multi(projections, n_projections, ys, x, norm_weight, norm_dtype, norm_eps, stream);
+    if (st == SWQ_OK) st = swq_deltanet_step(l, qkvz, ba, state, state_bytes, position, y, stream);
+    if (st == SWQ_OK) st = swq_encode_gemv(out_proj, 0, 0, 0, 0, y, 0, out, 0, stream);
+    return st;
+}

@@ -15,6 +15,9 @@ inline int hip_status(hipError_t e) { return e == hipSuccess ? SWQ_OK : SWQ_ERR_
 
 inline int launch_status() { return hip_status(hipGetLastError()); }
 
+// Intermediate vectors of one call's scratch buffer start at 256-byte boundaries.
+inline int64_t pad_floats(int64_t n) { return (n + 63) / 64 * 64; }
+
 inline int scale_bytes(int stype) { return stype == SWQ_F32 ? 4 : 2; }
 
 inline int ilog2_exact(int v) {

@@ -10,7 +10,7 @@ import ctypes
 
 from . import _lib
 from ._lib import SWQ_DELTA_INTERLEAVED, SWQ_DELTA_SPLIT, DeltaNetLayer, check
-from .engine import GPULinear, HipEngine, _stream_handle, _torch
+from .engine import DescArray, GPULinear, HipEngine, _norm_arg, _stream_handle, _torch
 
 
 class DeltaNetGPU:
@@ -41,6 +41,8 @@ class DeltaNetGPU:
             num_key_heads=nk, num_value_heads=nv, key_head_dim=dk, value_head_dim=dv, conv_kernel=conv_kernel,
             layout=layout, norm_eps=eps, reserved=0, conv_weight=self.conv_weight.data_ptr(),
             a_log=self.a_log.data_ptr(), dt_bias=self.dt_bias.data_ptr(), norm_weight=self.norm_weight.data_ptr())
+        self._projs = DescArray()
+        self._scratch = self.lib.swq_deltanet_scratch_floats(ctypes.byref(self._c))
 
     @property
     def state_bytes(self) -> int:
@@ -80,18 +82,14 @@ class DeltaNetGPU:
         """x [H] f32 -> the block's output [H]: the input projections in one
         launch (with norm_weight, x is the un-normalised hidden state and the
         input RMSNorm runs inside that launch), the step, out_proj."""
-        torch = _torch()
-        dev = x.device
-        qkvz = torch.empty(self.conv_dim + self.value_dim, dtype=torch.float32, device=dev)
-        ba = torch.empty(2 * self.nv, dtype=torch.float32, device=dev)
-        if self.layout == SWQ_DELTA_INTERLEAVED:
-            ys = [qkvz, ba]
-        else:
-            ys = [qkvz.data_ptr(), qkvz.data_ptr() + 4 * self.conv_dim, ba.data_ptr(), ba.data_ptr() + 4 * self.nv]
-        engine.encode_gemv_multi(list(self.projections), x, ys, norm_weight=norm_weight, eps=eps, stream=stream)
-        y = self.step(qkvz, ba, state, position, stream=stream)
-        r = torch.empty(self.out_proj.out_dim, dtype=torch.float32, device=dev)
-        engine.encode_gemv(self.out_proj, y, r, stream=stream)
+        empty, f32, dev = _torch().empty, _torch().float32, x.device
+        scratch = empty(self._scratch, dtype=f32, device=dev)
+        r = empty(self.out_proj.out_dim, dtype=f32, device=dev)
+        wdt, wptr = _norm_arg(norm_weight)
+        check(self.lib.swq_deltanet_token(
+            ctypes.byref(self._c), self._projs.of(self.projections), len(self.projections), self.out_proj.desc(),
+            x.data_ptr(), wptr, wdt, eps, state.data_ptr(), state.numel(), position, scratch.data_ptr(), self._scratch,
+            r.data_ptr(), _stream_handle(stream)), "deltanet_token")
         return r
 
 

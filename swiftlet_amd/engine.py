@@ -26,11 +26,36 @@ def _torch():
     return torch
 
 
-def _stream_handle(stream) -> ctypes.c_void_p:
+def _stream_handle(stream) -> int:
+    """The raw stream of a torch stream, or of the current one; without building a torch stream
+    object for the latter, which costs a launch's host time again."""
+    if stream is not None:
+        return stream.cuda_stream
+    cuda = _torch().cuda
+    return _torch()._C._cuda_getCurrentRawStream(cuda.current_device())
+
+
+def _norm_arg(weight):
+    """(dtype code, address) of a norm weight, or those of none."""
+    if weight is None:
+        return SWQ_F32, None
     torch = _torch()
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return {torch.float32: SWQ_F32, torch.float16: SWQ_F16, torch.bfloat16: SWQ_BF16}[weight.dtype], weight.data_ptr()
+
+
+class DescArray:
+    """The descriptors of several linears as one C array, rebuilt when one of them changed."""
+
+    def __init__(self):
+        self._last = ((), None)  # one tuple, so that threads see matching parts
+
+    def of(self, lins):
+        descs = tuple([l.desc() for l in lins])
+        last, arr = self._last
+        if len(descs) != len(last) or any([a is not b for a, b in zip(descs, last)]):
+            arr = (QLinear * len(descs))(*descs)
+            self._last = (descs, arr)
+        return arr
 
 
 def to_device_bytes(arr: np.ndarray, device="cuda"):
@@ -58,6 +83,27 @@ class GPULinear:
         self.w_off, self.s_off, self.b_off = w_off, s_off, b_off
         self.expert_stride_w, self.expert_stride_sb = expert_stride_w, expert_stride_sb
         self.num_experts = num_experts
+
+    # desc()'s last result with what it was made from, and a count of the fields set so far
+    _desc, _sets = None, 0
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        object.__setattr__(self, "_sets", self._sets + 1)
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_desc"}  # a C struct does not pickle
+
+    def desc(self) -> QLinear:
+        """The descriptor, shared between calls and not to be written: rebuilt when a field was
+        set or a tensor's storage moved, else the same object (building one costs ~3 us of host
+        time, as much as a launch)."""
+        made_from = (self._sets, self.w.data_ptr(), self.scales.data_ptr(), self.biases.data_ptr())
+        d = self._desc
+        if d is None or d[1] != made_from:
+            d = (self.c(), made_from)
+            object.__setattr__(self, "_desc", d)
+        return d[0]
 
     @property
     def matrix_bytes(self) -> int:
@@ -126,8 +172,7 @@ class HipEngine:
                     s_extra: int = 0, b_extra: int = 0, x_off: int = 0, y_off: int = 0, stream=None):
         torch = _torch()
         assert x.dtype == torch.float32 and y.dtype == torch.float32
-        c = lin.c()
-        check(self.lib.swq_encode_gemv(ctypes.byref(c), rows or 0, w_extra, s_extra, b_extra,
+        check(self.lib.swq_encode_gemv(ctypes.byref(lin.desc()), rows or 0, w_extra, s_extra, b_extra,
                                        x.data_ptr(), x_off, y.data_ptr(), y_off,
                                        _stream_handle(stream)), "encode_gemv")
 
@@ -136,14 +181,10 @@ class HipEngine:
         """ys[i] = W_i x (x: f32 device vector; ys: f32 device tensors or raw
         device addresses); with norm_weight, x is replaced by rmsnorm(x) *
         norm_weight inside the kernel."""
-        torch = _torch()
         n = len(lins)
-        arr = (QLinear * n)(*[l.c() for l in lins])
+        arr = (QLinear * n)(*[l.desc() for l in lins])
         ptrs = (ctypes.c_void_p * n)(*[y if isinstance(y, int) else y.data_ptr() for y in ys])
-        wdt, wptr = SWQ_F32, None
-        if norm_weight is not None:
-            wdt = {torch.float32: SWQ_F32, torch.float16: SWQ_F16, torch.bfloat16: SWQ_BF16}[norm_weight.dtype]
-            wptr = norm_weight.data_ptr()
+        wdt, wptr = _norm_arg(norm_weight)
         check(self.lib.swq_encode_gemv_multi(arr, n, ptrs, x.data_ptr(), wptr, wdt, eps, _stream_handle(stream)),
               "encode_gemv_multi")
 
@@ -192,18 +233,29 @@ class HipEngine:
         torch = _torch()
         dev = logits.device
         vocab = logits.numel()
+        if stream is not None and stream != torch.cuda.current_stream():
+            with torch.cuda.stream(stream):
+                return self.sample(logits, temperature, top_k, top_p, presence, frequency, seen, banned, u, ws)
         if ws is None:
             ws = self.new_sample_workspace(vocab, dev)
-        seen = seen or {}
-        ids = torch.tensor(list(seen.keys()) or [0], dtype=torch.int32, device=dev)
-        cnt = torch.tensor(list(seen.values()) or [0], dtype=torch.int32, device=dev)
-        ban = torch.tensor(list(banned) or [0], dtype=torch.int32, device=dev)
-        out = torch.empty(1, dtype=torch.int32, device=dev)
+        seen, banned = seen or {}, list(banned)
+        ids = cnt = ban = None
+        if seen or banned:
+            # ids, counts and banned ids in one copy, from pinned memory so that it is only
+            # enqueued: the caller's earlier work on the stream may still run
+            lists = torch.tensor([*seen.keys(), *seen.values(), *banned], dtype=torch.int32, pin_memory=True)
+            lists = lists.to(dev, non_blocking=True)
+            ids = lists.data_ptr()
+            cnt = ids + 4 * len(seen)
+            ban = cnt + 4 * len(seen)
+        # the kernel writes the token to host memory; reading it back takes a wait and no copy
+        out = torch.empty(1, dtype=torch.int32, pin_memory=True)
         opt = _lib.SampleOptions(temperature, top_k, top_p, presence, frequency)
-        check(self.lib.swq_sample(logits.data_ptr(), vocab, ctypes.byref(opt), ids.data_ptr(), cnt.data_ptr(),
-                                  len(seen), ban.data_ptr(), len(banned), u, out.data_ptr(), ws.data_ptr(),
-                                  ws.numel(), _stream_handle(stream)), "sample")
-        return int(out.item())
+        check(self.lib.swq_sample(logits.data_ptr(), vocab, ctypes.byref(opt), ids, cnt, len(seen), ban,
+                                  len(banned), u, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                  _stream_handle(None)), "sample")
+        torch.cuda.current_stream().synchronize()
+        return int(out)
 
     # Checkpoint.moduleWeightSlice (Checkpoint.swift:148-155): rows of the
     # flattened [experts*out, in] weight as fp32.

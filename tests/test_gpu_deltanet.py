@@ -209,3 +209,49 @@ def test_tiny_q35_model_with_device_deltanet_matches_mlx():
     assert np.abs(logits - fx["logits"][0]).max() < 0.05
     want = json.loads((G / "tiny_forward_q35.json").read_text())["greedy_next_tokens"]
     assert np.argmax(logits, axis=-1).tolist() == want
+
+
+def test_token_entry_equals_its_launches():
+    """forward_token's one native call against the launches it stands for, in both layouts, and
+    after a weight of a projection was replaced (its descriptor is kept between calls)."""
+    import torch
+    from swiftlet_amd._lib import SWQ_DELTA_INTERLEAVED, SWQ_DELTA_SPLIT
+    from swiftlet_amd.attention import AttentionGPU
+    from swiftlet_amd.engine import HipEngine
+    from swiftlet_amd.moe import synth_linear
+    eng = HipEngine()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    lin = lambda seed, rows, cols: synth_linear(seed, 0, "router", None, rows, cols, 4, 64)  # noqa: E731
+    nk, nv, dk, dv, K, H = 2, 4, 16, 32, 4, 256
+    conv, val = 2 * nk * dk + nv * dv, nv * dv
+    x, w = r(H), 1 + 0.1 * r(H)
+    for layout, rows in ((SWQ_DELTA_SPLIT, (conv, val, nv, nv)), (SWQ_DELTA_INTERLEAVED, (conv + val, 2 * nv))):
+        blk = DeltaNetGPU(nk, nv, dk, dv, K, layout, 1e-6, r(conv * K), r(nv), r(nv), r(dv),
+                          projections=[lin(i, n, H) for i, n in enumerate(rows)], out_proj=lin(9, H, val))
+        for step in range(2):
+            state = blk.new_state()
+            qkvz, ba = torch.empty(conv + val, device="cuda"), torch.empty(2 * nv, device="cuda")
+            ys = [qkvz[:conv], qkvz[conv:], ba[:nv], ba[nv:]] if layout == SWQ_DELTA_SPLIT else [qkvz, ba]
+            eng.encode_gemv_multi(list(blk.projections), x, ys, norm_weight=w)
+            want = torch.empty(H, device="cuda")
+            eng.encode_gemv(blk.out_proj, blk.step(qkvz, ba, state, 5), want)
+            state2 = blk.new_state()
+            got = blk.forward_token(eng, x, state2, 5, norm_weight=w)
+            assert torch.equal(got, want) and torch.equal(state, state2), (layout, step)
+            if step:
+                assert not torch.equal(got, first)
+            first = got
+            blk.projections[0].w = lin(77, rows[0], H).w
+    heads, kvh, hd = 4, 2, 32
+    att = AttentionGPU(heads, kvh, hd, 8, 1e4, 1e-6, 40, r(hd), r(hd),
+                       projections=[lin(20 + i, n, H) for i, n in enumerate((2 * heads * hd, kvh * hd, kvh * hd))],
+                       o_proj=lin(30, H, heads * hd))
+    cache, cache2, ws = att.new_cache(), att.new_cache(), att.new_workspace()
+    for pos in range(3):
+        q, k, v = (torch.empty(p.out_dim, device="cuda") for p in att.projections)
+        eng.encode_gemv_multi(list(att.projections), x, [q, k, v], norm_weight=w)
+        want = torch.empty(H, device="cuda")
+        eng.encode_gemv(att.o_proj, att.step(q, k, v, cache, ws, pos), want)
+        assert torch.equal(att.forward_token(eng, x, cache2, ws, pos, norm_weight=w), want), pos
+    assert torch.equal(cache, cache2)
