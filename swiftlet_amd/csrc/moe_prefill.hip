@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/swq_bench.h"
 #include "moe_host.hpp"
@@ -146,14 +147,29 @@ __device__ __forceinline__ u32x4_t nibble_order(u32x4_t d) {
     return o;
 }
 
+// (v & mask) | magic, as one v_and_or_b32 by way of operands the compiler cannot fold into
+// literals (mask in a scalar register, magic in a vector one: one scalar operand is allowed).
+// Not the instruction in inline asm: the compiler cannot see that such an instruction writes a
+// register that a matrix product issued just before still reads or will write, and puts no wait
+// between them.
+struct CodeMask {
+    uint32_t mask, magic;
+    __device__ __forceinline__ CodeMask() : mask(0x00780078u), magic(0x41804180u) {
+        asm("" : "+s"(mask));
+        asm("" : "+v"(magic));
+    }
+    __device__ __forceinline__ uint32_t operator()(uint32_t v) const { return (v & mask) | magic; }
+};
+
 // 8 codes of one 4-bit word as bf16 (16 + q: the code in the top four
 // mantissa bits of 16.0), in nibble_order.
 __device__ __forceinline__ u32x4_t codes_q4(uint32_t w) {
+    const CodeMask m;
     u32x4_t o;
-    o[0] = and_or(w << 3, 0x00780078u, 0x41804180u);
-    o[1] = and_or(w >> 1, 0x00780078u, 0x41804180u);
-    o[2] = and_or(w >> 5, 0x00780078u, 0x41804180u);
-    o[3] = and_or(w >> 9, 0x00780078u, 0x41804180u);
+    o[0] = m(w << 3);
+    o[1] = m(w >> 1);
+    o[2] = m(w >> 5);
+    o[3] = m(w >> 9);
     return o;
 }
 
@@ -1080,6 +1096,212 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 }
 
 // ---------------------------------------------------------------------------
+// the ring GEMM over tiles of at most 16 rows (gate/up, down of few tokens)
+
+constexpr int kThinRows = 16;
+
+// pf_gemm_dma for tiles of at most kThinRows rows, bit for bit.  With few rows
+// the codes are the work, and a ring of single 64-input groups reads them in
+// 32-byte pieces and pays a barrier and an LDS round trip per group.  Here a
+// ring stage is 128 bytes of every code row, whole cache lines (four groups of
+// 4-bit codes, two of 8-bit ones), next to the 16 activation rows of those
+// groups; S stages.  Row r's 16-byte chunk c sits in slot c ^ (r & 7) of its
+// 128 bytes, codes and activations alike.
+//
+// Bound: the codes' bytes, then (one token) the latency of a workgroup's eight
+// stages.  gate/up and down of 256 experts top-8, 4-bit, us: one token 20.9 ->
+// 14.1 and 10.2 -> 6.2; 16 tokens (~105 experts, 120 + 61 MB) 46.5 -> 33.7 and
+// 29.6 -> 24.6.  Measured beside it, bit for bit the same: every code of a wave in registers with K split over four
+// waves, 60 and 35 us at 16 tokens; one-wave workgroups, 256-byte row pieces
+// in 32 KB of LDS, 57 and 45; the single-group ring with 16-row activation
+// slots six groups deep, 42 and 26.
+template <int BITS, int ST, int NPL, int EPI, int S>
+__global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
+    constexpr int WAVES = 4, GPS = BITS == 4 ? 4 : 2;  // groups per stage
+    constexpr int A_GROUP = NPL * kThinRows * 128, A_STAGE = GPS * A_GROUP;
+    constexpr int B_WAVE = 4096, B_STAGE = WAVES * B_WAVE;
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring_a[S * A_STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring_b[S * B_STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t s_xs[kThinRows * 128];
+    __shared__ float s_red[EPI == kEpiSwiGLU ? WAVES * kThinRows : 1];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, kg = lane >> 4;
+    const int xcd = blockIdx.x & (kXcds - 1), q = blockIdx.x >> 3;
+    const int ti = (q / a.nblk) * kXcds + xcd, nb = q % a.nblk;
+    const int n_tiles = *a.n_tiles;
+    const Tile t = a.tiles[min(ti, a.max_tiles - 1)];
+    if (ti >= n_tiles) return;
+    const int expert = t.expert, row0 = t.row0, rows = t.rows;
+    // a table from a workspace that skipped swq_moe_workspace_init
+    if (expert < 0 || expert > a.E || rows <= 0 || rows > kThinRows || row0 < 0 || row0 + rows > a.rows_total) return;
+    const bool shared = expert == a.E;
+    const int N = shared ? a.Nsh : a.N;
+    const int NG = (shared ? a.Ksh : a.K) / kGroupK, NS = (NG + GPS - 1) / GPS;
+    const int wcol = nb * a.col_block + wave * a.col_wave;
+    const bool active = wcol < N;
+
+    const uint8_t *wbase[2], *sbase[2], *bbase[2];
+    int64_t srow[2];
+    int col[2];
+    int row_bytes = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const QMat &m = shared ? a.sh[j] : a.m[j];
+        col[j] = wcol + j * a.col_op + n;
+        const int64_t eoff_w = shared ? 0 : static_cast<int64_t>(expert) * m.stride_w;
+        const int64_t eoff_s = shared ? 0 : static_cast<int64_t>(expert) * m.stride_sb;
+        wbase[j] = m.w + eoff_w;
+        sbase[j] = m.s + eoff_s;
+        bbase[j] = m.b + eoff_s;
+        srow[j] = static_cast<int64_t>(min(col[j], N - 1)) * m.gpr;
+        row_bytes = m.row_bytes;
+    }
+    // copy i of the wave's codes: rows 8 i + lane / 8 of the two operands (0..31)
+    const int l8 = lane >> 3, off8 = 16 * ((lane & 7) ^ l8);
+    const uint8_t *bsrc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int j = i >> 1, R = min(wcol + j * a.col_op + 8 * (i & 1) + l8, N - 1);
+        bsrc[i] = (j ? wbase[1] : wbase[0]) + static_cast<int64_t>(R) * row_bytes;
+    }
+    // the wave's activation copies: 4-bit: group `wave` of the stage, both 8-row slabs; 8-bit:
+    // group wave / 2, slab wave % 2; every plane.  Rows past the tile are not fetched (lane 0
+    // always is), slabs past it not copied.
+    const int slabs = rows > 8 ? 2 : 1;
+    const int au = BITS == 4 ? wave : wave >> 1, as0 = BITS == 4 ? 0 : wave & 1;
+    const int as1 = BITS == 4 ? slabs : min(as0 + 1, slabs);  // slabs [as0, as1)
+    const int na = max(0, as1 - as0) * NPL;
+    const uint8_t *asrc[2], *xsrc[2];
+    bool fetch[2];
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+        const int r = 8 * sl + l8, rr = r < rows ? r : 0;
+        fetch[sl] = r < rows || lane == 0;
+        const int64_t sr = min(max(a.row_src ? a.row_src[row0 + rr] : row0 + rr, 0), a.a_rows - 1);
+        asrc[sl] = reinterpret_cast<const uint8_t *>(2 * sr * a.a_ld + off8);  // an offset, of either plane
+        xsrc[sl] = reinterpret_cast<const uint8_t *>(a.xs_in + sr * a.xs_ld) + off8;
+    }
+    const uint32_t ring_a = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_ring_a));
+    const uint32_t ring_b = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_ring_b));
+
+    // biases and scales, then the group sums, ahead of every ring load
+    BiasBS<ST> bi;
+    load_bias_bs<ST>(bi, sbase, bbase, srow, NG, kg);
+    if (wave < slabs) {
+        const uint32_t d = __builtin_amdgcn_readfirstlane(
+            static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_xs)) + wave * 1024);
+        if (wave ? fetch[1] : fetch[0]) dma16(wave ? xsrc[1] : xsrc[0], d);
+    }
+    auto issue = [&](int slot, int st) {
+        const uint32_t b = __builtin_amdgcn_readfirstlane(ring_b + slot * B_STAGE + wave * B_WAVE);
+        const int off = min(128 * st + off8, row_bytes - 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dma16(bsrc[i] + off, b + i * 1024);
+        const uint32_t d0 = ring_a + slot * A_STAGE + au * A_GROUP;
+        const int g = min(st * GPS + au, NG - 1);
+#pragma unroll
+        for (int sl = 0; sl < 2; ++sl) {
+            if (sl < as0 || sl >= as1) continue;
+#pragma unroll
+            for (int p = 0; p < NPL; ++p) {
+                const uint32_t d = __builtin_amdgcn_readfirstlane(d0 + (p * kThinRows + 8 * sl) * 128);
+                const uint8_t *base = static_cast<const uint8_t *>(p ? a.a1 : a.a0) + kGroupK * 2 * g;
+                if (fetch[sl]) dma16(base + reinterpret_cast<uintptr_t>(asrc[sl]), d);
+            }
+        }
+    };
+
+    f32x4_t acc[1][2];
+    acc[0][0] = acc[0][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int x7 = n & 7;
+    // the first CNT groups of a stage, with no branch between them
+    auto compute = [&](auto CNT, int slot, int st) {
+        const uint8_t *al = s_ring_a + slot * A_STAGE + n * 128;
+        const uint8_t *bl = s_ring_b + slot * B_STAGE + wave * B_WAVE + n * 128;
+#pragma unroll
+        for (int u = 0; u < CNT(); ++u) {
+            const int g = st * GPS + u;
+            float sc[2];
+            if constexpr (ST == SWQ_F32) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) sc[j] = reinterpret_cast<const float *>(sbase[j])[srow[j] + g];
+            } else {
+                scales_from_bs<ST>(bi, g, n, sc);
+            }
+            const int c0 = ((2 * kg) ^ x7) * 16, c1 = ((2 * kg + 1) ^ x7) * 16;
+            u32x4_t av[NPL][2];
+#pragma unroll
+            for (int p = 0; p < NPL; ++p) {
+                av[p][0] = *reinterpret_cast<const u32x4_t *>(al + u * A_GROUP + p * kThinRows * 128 + c0);
+                av[p][1] = *reinterpret_cast<const u32x4_t *>(al + u * A_GROUP + p * kThinRows * 128 + c1);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                u32x4_t bq[2];
+                if constexpr (BITS == 4) {
+                    const uint2 w = *reinterpret_cast<const uint2 *>(
+                        bl + j * 2048 + 16 * ((2 * u + (kg >> 1)) ^ x7) + 8 * (kg & 1));
+                    bq[0] = codes_q4(w.x);
+                    bq[1] = codes_q4(w.y);
+                } else {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(bl + j * 2048 + 16 * ((4 * u + kg) ^ x7));
+                    bq[0] = codes_q8(w.x, w.y);
+                    bq[1] = codes_q8(w.z, w.w);
+                }
+                f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < NPL; ++p)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) c = mfma(av[p][i], bq[i], c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[0][j][e] = fmaf(sc[j], c[e], acc[0][j][e]);
+            }
+        }
+    };
+
+    // ---- the ring: stages 0 .. S-2 first; at stage st, wait until it has
+    // landed (the newest min(S - 2, NS - 1 - st) stages may be in flight, 4 + na
+    // copies each), refill the slot that stage st - 1 used, compute
+#pragma unroll
+    for (int st = 0; st < S - 1; ++st)
+        if (st < NS) issue(st, st);
+    int slot = 0, prev = S - 1;
+#pragma unroll 1
+    for (int st = 0; st < NS; ++st) {
+        static_assert(S == 2 || S == 3, "wait counts");
+        if (S == 3 && st + 1 < NS) ring_wait_sel<4, 5, 6, 7, 8>(na);
+        else ring_wait<0>();
+        if constexpr (ST != SWQ_F32) {
+            // the scale words have landed (they are older than the ring): one wait for them
+            // here, not one in every pass (as in pf_gemm_dma)
+            if (st == 0) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bi.s[j][i]));
+            }
+        }
+        if (st + S - 1 < NS) issue(prev, st + S - 1);
+        // (group counts are even, so a short stage of four has two)
+        if (GPS == 2 || (st + 1) * GPS <= NG) compute(std::integral_constant<int, GPS>{}, slot, st);
+        else compute(std::integral_constant<int, 2>{}, slot, st);
+        prev = slot;
+        slot = slot + 1 == S ? 0 : slot + 1;
+    }
+
+    if (active) {
+        const uint8_t *xr = s_xs + n * 128;
+        const float4 x0 = *reinterpret_cast<const float4 *>(xr + 16 * ((2 * kg) ^ x7));
+        const float4 x1 = *reinterpret_cast<const float4 *>(xr + 16 * ((2 * kg + 1) ^ x7));
+        const float xv[1][8] = {{x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}};
+        bias_term_bs<BITS, ST, 1>(acc, bi, xv, NG, rows, kg);
+    }
+    epilogue<EPI, 1, WAVES>(acc, a, col, N, active, row0, rows, nb, s_red);
+}
+
+// ---------------------------------------------------------------------------
 // routing and grouping
 
 constexpr int kMaxLogitSlices = 16;  // router K slices (partial logit rows per token): H <= 4096
@@ -1099,6 +1321,7 @@ struct RouteArgs {
     Tile *tiles;
     int32_t *n_tiles;
     int32_t T, E, K, H, norm, has_shared;
+    int32_t tile_rows;        // most rows of a tile: kTileRows or kThinRows
     int32_t lslices;
     int64_t lslice;           // elements between slices
 };
@@ -1166,7 +1389,7 @@ __device__ void group_pairs(const RouteArgs &a) {
     constexpr int kHeldIds = 4096 / NT;  // every id of 512 tokens x top-8
     constexpr int kBatch = 8;  // ids per thread per pass past the held ones, all in flight at once
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int P = a.T * a.K;
+    const int P = a.T * a.K, cap = a.tile_rows;
     int held[kHeldIds];
 #pragma unroll
     for (int u = 0; u < kHeldIds; ++u) held[u] = a.ids[min(tid + u * NT, P - 1)];
@@ -1192,7 +1415,7 @@ __device__ void group_pairs(const RouteArgs &a) {
     for (int i = 0; i < EPT; ++i) {
         const int e = tid * EPT + i;
         cnt[i] = e < a.E ? s_cnt[e] : 0;
-        tl[i] = (cnt[i] + kTileRows - 1) / kTileRows;
+        tl[i] = (cnt[i] + cap - 1) / cap;
         csum += cnt[i];
         tsum += tl[i];
     }
@@ -1206,17 +1429,17 @@ __device__ void group_pairs(const RouteArgs &a) {
     // The tile table in decreasing row count (the GEMMs start the heaviest
     // tiles first, so the light ones fill in at the end): tiles per row
     // count, their first slots, then each tile into the next slot of its count.
-    const int sh_tiles = a.has_shared ? (a.T + kTileRows - 1) / kTileRows : 0;
+    const int sh_tiles = a.has_shared ? (a.T + cap - 1) / cap : 0;
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
         if (tid * EPT + i < a.E && cnt[i] > 0) {
-            if (cnt[i] >= kTileRows) atomicAdd(&s_rows[kTileRows], cnt[i] / kTileRows);
-            if (cnt[i] % kTileRows) atomicAdd(&s_rows[cnt[i] % kTileRows], 1);
+            if (cnt[i] >= cap) atomicAdd(&s_rows[cap], cnt[i] / cap);
+            if (cnt[i] % cap) atomicAdd(&s_rows[cnt[i] % cap], 1);
         }
     }
     if (tid == 0 && sh_tiles > 0) {
-        if (a.T >= kTileRows) atomicAdd(&s_rows[kTileRows], a.T / kTileRows);
-        if (a.T % kTileRows) atomicAdd(&s_rows[a.T % kTileRows], 1);
+        if (a.T >= cap) atomicAdd(&s_rows[cap], a.T / cap);
+        if (a.T % cap) atomicAdd(&s_rows[a.T % cap], 1);
     }
     __syncthreads();
     int c0 = cinc - csum, routed_tiles = 0;
@@ -1239,15 +1462,15 @@ __device__ void group_pairs(const RouteArgs &a) {
         if (e < a.E) {
             s_cnt[e] = c0;  // each thread rewrites only its own experts
             for (int q = 0; q < tl[i]; ++q) {
-                const int rows = min(kTileRows, cnt[i] - q * kTileRows);
-                a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{e, c0 + q * kTileRows, rows, 0};
+                const int rows = min(cap, cnt[i] - q * cap);
+                a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{e, c0 + q * cap, rows, 0};
             }
         }
         c0 += cnt[i];
     }
     for (int q = tid; q < sh_tiles; q += NT) {
-        const int rows = min(kTileRows, a.T - q * kTileRows);
-        a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{a.E, P + q * kTileRows, rows, 0};
+        const int rows = min(cap, a.T - q * cap);
+        a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{a.E, P + q * cap, rows, 0};
     }
     if (tid == 0) *a.n_tiles = routed_tiles + sh_tiles;
     __syncthreads();
@@ -1438,6 +1661,18 @@ __global__ __launch_bounds__(kPfThreads) void pf_combine(const CombineArgs a) {
 // blocks x slices fill the device and a slice's loads are one round trip.
 int router_kslices(int H) { return (H / kGroupK + kBlockG - 1) / kBlockG; }
 
+// Tiles of at most kThinRows rows, for pf_gemm_thin, while the experts see few rows each: up to
+// kThinAvgRows on average.  The layer's time with 64-row and with 16-row tiles, us (bf16 x):
+//   tokens                    24     64    128    192    256    512
+//   256 experts top-8, 4-bit  84/74 120/103 135/121 149/138 159/153 194/212
+//   256 experts top-8, 8-bit 112/103 155/131 185/166 200/185 213/202 247/276
+//   512 experts top-10, 4-bit 113/98 161/139 196/171 221/200 237/223 309/316
+// (f32 x at 256 tokens, 4-bit: 165/170.)
+constexpr int kThinAvgRows = 6;
+bool thin_tiles(const swq_moe_layer *l, int T) {
+    return T <= kThinRows || static_cast<int64_t>(T) * l->top_k <= static_cast<int64_t>(kThinAvgRows) * l->num_experts;
+}
+
 struct PfLayout {
     size_t header, logits, sg, ids, wts, pos, tok, tiles, xs_x, xs_h, xa0, xa1, h_hi, h_lo, y, total;
     int max_tiles, Ih, xs_ld_x, xs_ld_h, kslices;
@@ -1454,8 +1689,9 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
     const size_t P = static_cast<size_t>(T) * l->top_k;
     const size_t rows = P + (l->has_shared ? T : 0);
     const int U = static_cast<int>(std::min<size_t>(P, static_cast<size_t>(l->num_experts)));
-    w.max_tiles = static_cast<int>((P + static_cast<size_t>(kTileRows - 1) * U) / kTileRows) +
-                  (l->has_shared ? (T + kTileRows - 1) / kTileRows : 0);
+    const int cap = thin_tiles(l, T) ? kThinRows : kTileRows;
+    w.max_tiles = static_cast<int>((P + static_cast<size_t>(cap - 1) * U) / cap) +
+                  (l->has_shared ? (T + cap - 1) / cap : 0);
     w.Ih = std::max(l->moe_intermediate, l->has_shared ? l->shared_intermediate : 0);
     w.header = take(256);  // [1] tile count
     w.kslices = router_kslices(l->hidden);
@@ -1601,6 +1837,32 @@ int launch_dma(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream_
     return launch_status();
 }
 
+// Ring stages of the thin GEMM: two, 43 to 68 KB of LDS and two or three
+// workgroups per CU; three stages measured 36 against 34 us for gate/up and 37
+// against 25 us for down (16 tokens, 256 experts top-8, 4-bit).
+constexpr int kThinStages = 2;
+
+template <int BITS, int NPL, int EPI>
+void launch_thin_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
+    constexpr int D = kThinStages;
+    const dim3 g(blocks), th(kPfThreads);
+    if (stype == SWQ_F16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F16, NPL, EPI, D>), g, th, 0, s, a);
+    else if (stype == SWQ_BF16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_BF16, NPL, EPI, D>), g, th, 0, s, a);
+    else hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F32, NPL, EPI, D>), g, th, 0, s, a);
+}
+
+// The thin GEMM over the tile table; sets the column steps and the grid of `a`.
+template <int NPL, int EPI>
+int launch_thin(const swq_qlinear &lin, GemmArgs &a, int max_tiles, int N, hipStream_t s) {
+    a.col_block = 4 * a.col_wave;
+    a.nblk = (N + a.col_block - 1) / a.col_block;
+    const int blocks = gemm_blocks(max_tiles, a.nblk);
+    if (blocks <= 0) return SWQ_OK;
+    if (lin.bits == 4) launch_thin_st<4, NPL, EPI>(lin.scales_type, a, blocks, s);
+    else launch_thin_st<8, NPL, EPI>(lin.scales_type, a, blocks, s);
+    return launch_status();
+}
+
 int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, void *out, int out_dtype,
                  int32_t *topk_ids, float *topk_weights, const float *logit_bias, void *ws, size_t ws_bytes,
                  int flags, int stage_mask, void *stream) {
@@ -1639,6 +1901,7 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
     float *xs_h = reinterpret_cast<float *>(wsb + wl.xs_h);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16x = x_dtype == SWQ_BF16;
+    const bool thin = thin_tiles(layer, T);
 
     // x planes for gate/up (nibble_order for 4-bit codes, hi/lo for fp32 x)
     // and the group sums of x: written by the router GEMM as it stages x
@@ -1700,6 +1963,7 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         r.H = H;
         r.norm = layer->norm_topk_prob ? 1 : 0;
         r.has_shared = layer->has_shared ? 1 : 0;
+        r.tile_rows = thin ? kThinRows : kTileRows;
         const int blocks = (T + kRouteWaves - 1) / kRouteWaves;
         if (bf16x) hipLaunchKernelGGL(pf_route<SWQ_BF16>, dim3(blocks), dim3(kRouteWaves * kWave), 0, s, r);
         else hipLaunchKernelGGL(pf_route<SWQ_F32>, dim3(blocks), dim3(kRouteWaves * kWave), 0, s, r);
@@ -1741,9 +2005,14 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.col_op = 0;
         g.nblk = (wl.Ih + g.col_block - 1) / g.col_block;
         g.max_tiles = wl.max_tiles;
-        const int blocks = gemm_blocks(wl.max_tiles, g.nblk);
-        st = bf16x ? launch_dma<1, kEpiSwiGLU>(layer->gate, g, blocks, s)
-                   : launch_dma<2, kEpiSwiGLU>(layer->gate, g, blocks, s);
+        if (thin) {
+            st = bf16x ? launch_thin<1, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, s)
+                       : launch_thin<2, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, s);
+        } else {
+            const int blocks = gemm_blocks(wl.max_tiles, g.nblk);
+            st = bf16x ? launch_dma<1, kEpiSwiGLU>(layer->gate, g, blocks, s)
+                       : launch_dma<2, kEpiSwiGLU>(layer->gate, g, blocks, s);
+        }
         if (st != SWQ_OK) return st;
     }
     // 4. down over the tiles
@@ -1771,8 +2040,9 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.col_op = 16;
         g.nblk = (H + g.col_block - 1) / g.col_block;
         g.max_tiles = wl.max_tiles;
-        const int blocks = gemm_blocks(wl.max_tiles, g.nblk);
-        if ((st = launch_dma<2, kEpiRows>(layer->down, g, blocks, s)) != SWQ_OK) return st;
+        if (thin) st = launch_thin<2, kEpiRows>(layer->down, g, wl.max_tiles, H, s);
+        else st = launch_dma<2, kEpiRows>(layer->down, g, gemm_blocks(wl.max_tiles, g.nblk), s);
+        if (st != SWQ_OK) return st;
     }
     // 5. weighted combine in pick order, then the gated shared expert
     if (stage_mask & 32) {

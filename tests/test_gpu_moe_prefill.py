@@ -277,3 +277,28 @@ def test_prefill_router_scales_two_bytes_past_a_word():
     assert torch.equal(ids, ref_ids)
     assert torch.equal(w, ref_w)
     assert torch.equal(out, ref_out)
+
+
+@pytest.mark.parametrize("H,I,Is,bits,x_dtype,f32_scales", [
+    (2048, 512, 512, 4, "bf16", False), (384, 384, 128, 4, "bf16", False), (128, 640, 256, 4, "f32", False),
+    (640, 128, 384, 8, "bf16", False), (256, 896, 0, 8, "f32", False), (384, 256, 128, 4, "bf16", True),
+    (256, 384, 128, 8, "f32", True)])
+def test_few_tokens_equal_many(H, I, Is, bits, x_dtype, f32_scales):
+    """The GEMM over 16-row tiles (up to six tokens per expert on average: 90 tokens of 60 experts,
+    top 4) gives the bits of the one over 64-row tiles: the rows of calls of 1, 8, 9, 16, 17 and 90
+    tokens equal those of a call of 91.  Group counts that fill its stages and ones that do not
+    (6, 10, 14 groups), both activation forms, 2- and 4-byte scales."""
+    import torch
+    shape = synth.MoEShape("few", H, 60, 4, I, Is, expert_bits=bits, router_bits=8, group=64, norm_topk_prob=True)
+    gpu = moe.synth_layer(shape, 4000 + H + I, 0)
+    if f32_scales:
+        gpu = helpers.widen_layer(gpu)
+    x, _ = _x(77 + H, 91, H)
+    if x_dtype == "f32":
+        x = x.float() * 1.1
+    print(f"few tokens: H {H} I {I} Is {Is} q{bits} x {x_dtype} f32 scales {f32_scales}", flush=True)
+    want, want_ids, want_w = gpu.prefill(x)
+    for T in (1, 8, 9, 16, 17, 90):
+        out, ids, w = gpu.prefill(x[:T].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want_ids[:T]) and torch.equal(w, want_w[:T]) and torch.equal(out, want[:T]), T
