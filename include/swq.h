@@ -460,7 +460,11 @@ int swq_moe_workspace_status(void *ws, size_t ws_bytes, int clear, void *stream)
  *   1. router GEMV + shared-gate GEMV + shared gate/up SwiGLU;
  *   2. top-k per token, the distinct experts, their gate/up SwiGLU rows for
  *      all their tokens, indexed by the device-resident ids;
- *   3. down projections + weighted combine + sigmoid-gated shared expert.
+ *   3. down projections + weighted combine + sigmoid-gated shared expert;
+ * or, from five tokens on where the experts are large enough, as
+ * swq_moe_prefill's launches (the pairs sorted by expert, matrix cores), if
+ * the prefill takes the layer, out is 16-byte aligned and the workspace holds
+ * swq_moe_decode_workspace_bytes(layer, batch).
  * x: [batch, hidden] of x_dtype (SWQ_F32 / SWQ_BF16).  out: [batch, hidden]
  * of out_dtype (SWQ_F32 / SWQ_BF16).  topk_ids [batch, top_k] int32 and
  * topk_weights [batch, top_k] f32 receive the routing (either may be NULL).

@@ -799,7 +799,7 @@ using namespace swq;
 
 extern "C" size_t swq_moe_decode_workspace_bytes(const swq_moe_layer *layer, int batch) {
     if (check_layer(layer, batch, SWQ_BF16) != SWQ_OK) return 0;
-    return decode_ws_bytes(layer, batch, false);
+    return decode_ws_bytes(layer, batch);
 }
 
 extern "C" int swq_moe_workspace_init(void *ws, size_t ws_bytes, void *stream) {
@@ -844,7 +844,8 @@ extern "C" int swq_moe_workspace_status(void *ws, size_t ws_bytes, int clear, vo
 
 // stage_mask: bits 0-2 run the staged kernels' stages; SWQ_STAGES_FUSED
 // runs the single-launch path (SWQ_ERR_LIMIT when this layer, batch or device
-// cannot); 0 picks the single launch when possible, else the three stages.
+// cannot); 0 picks the grouped path for wide batches, the single launch when
+// possible, else the three stages.
 static int moe_decode_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int batch, void *out,
                            int out_dtype, int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes,
                            int flags, int stage_mask, void *stream, bool max_layout = false) {
@@ -865,6 +866,12 @@ static int moe_decode_impl(const swq_moe_layer *layer, const void *x, int x_dtyp
     if (reinterpret_cast<uintptr_t>(ws) % 256 != 0) return SWQ_ERR_MISALIGNED;
 
     uint8_t *wsb = static_cast<uint8_t *>(ws);
+    if (stage_mask == 0 && grouped_pays(layer, x_dtype, batch)) {
+        const size_t n = grouped_ws_bytes(layer, batch);
+        if (n > 0 && grouped_ws_base(fl) + n <= ws_bytes && reinterpret_cast<uintptr_t>(out) % 16 == 0)
+            return grouped_decode(layer, x, x_dtype, batch, out, out_dtype, topk_ids, topk_weights,
+                                  wsb + grouped_ws_base(fl), n, flags, static_cast<hipStream_t>(stream));
+    }
     MoEArgs a{};
     a.router = make_qmat(&layer->router);
     a.gate = make_qmat(&layer->gate);
@@ -993,7 +1000,7 @@ extern "C" int swq_moe_decode_norm(const swq_moe_layer *layer, const float *h, c
         reinterpret_cast<uintptr_t>(norm_weight) % (norm_dtype == SWQ_F32 ? 4 : 2) != 0)
         return SWQ_ERR_MISALIGNED;
     const FusedLayout fl = fused_layout(layer, false);
-    if (!ws || ws_bytes < decode_ws_bytes(layer, 1, false)) return SWQ_ERR_WORKSPACE;
+    if (!ws || ws_bytes < decode_ws_bytes(layer, 1)) return SWQ_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(ws) % 256 != 0) return SWQ_ERR_MISALIGNED;
     const FusedPrenorm pn{h, residual, norm_weight, norm_dtype, norm_eps};
     bool taken = false;
@@ -1094,7 +1101,7 @@ extern "C" int swq_moe_decode_noalloc(const swq_moe_layer *layer, const void *x,
                                       void *stream) {
     const int st0 = check_layer(layer, batch, SWQ_BF16);
     if (st0 != SWQ_OK) return st0;
-    if (decode_ws_bytes(layer, batch, true) > kScratchBytes) return SWQ_ERR_LIMIT;
+    if (staged_ws_bytes(layer, batch, true) > kScratchBytes) return SWQ_ERR_LIMIT;
     uint8_t *ws = nullptr;
     const int st = scratch_for_device(static_cast<hipStream_t>(stream), &ws);
     if (st != SWQ_OK) return st;

@@ -2,6 +2,8 @@
 // the staged and the single-launch paths.
 #pragma once
 
+#include <algorithm>
+
 #include "internal.hpp"
 
 namespace swq {
@@ -144,9 +146,43 @@ inline FusedLayout fused_layout(const swq_moe_layer *l, bool max_shape) {
     return f;
 }
 
-// Bytes of the whole decode workspace for `batch` tokens.
-inline size_t decode_ws_bytes(const swq_moe_layer *l, int batch, bool max_shape) {
+// Bytes of a decode workspace without the grouped path's region.
+inline size_t staged_ws_bytes(const swq_moe_layer *l, int batch, bool max_shape) {
     return ws_layout(l, batch, fused_layout(l, max_shape).total).total;
+}
+
+// The grouped path of wide batches (moe_prefill.hip): the tokens' pairs sorted
+// by expert and each expert's rows contracted on the matrix cores, as a prefill
+// of `batch` tokens.  It works in the staged path's place, after the single
+// launch's regions, and keeps nothing from call to call.  grouped_ws_bytes: 0
+// when the prefill does not take the layer.
+size_t grouped_ws_bytes(const swq_moe_layer *l, int batch);
+int grouped_decode(const swq_moe_layer *layer, const void *x, int x_dtype, int batch, void *out, int out_dtype,
+                   int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes, int flags, hipStream_t stream);
+inline size_t grouped_ws_base(const FusedLayout &f) { return align256(f.total); }
+
+// Where the grouped path is the faster one: the three launches' time goes with
+// the codes that every (token, pick) pair multiplies, the grouped path's with
+// the distinct experts' bytes on top of its six launches.  us for three
+// launches / grouped, 256 experts top-8 (3.1 M codes a pair):
+//   batch             5      6      7      8      11      16
+//   4-bit, bf16 x   58/55  65/55  72/58  78/59  103/68  135/79
+//   4-bit, f32 x    65/57  74/58  82/60  90/61  116/74  157/86
+//   8-bit, bf16 x   54/62  60/63  68/67  71/70   91/82  121/104
+//   8-bit, f32 x    59/64  67/64  75/68  81/72  106/86  141/107
+// and 512 experts top-10, 4-bit, bf16 x: 71/61 at 5, 170/98 at 16.
+constexpr int kGroupedMinBatch = 5;
+inline bool grouped_pays(const swq_moe_layer *l, int x_dtype, int batch) {
+    const double codes = 3.0 * batch * l->top_k * l->hidden * l->moe_intermediate;
+    return batch >= kGroupedMinBatch && codes >= (l->gate.bits == 4 ? 120e6 : (x_dtype == SWQ_F32 ? 150e6 : 175e6));
+}
+
+// Bytes of the whole decode workspace for `batch` tokens: whatever batch up to
+// that and whatever activations the calls bring.
+inline size_t decode_ws_bytes(const swq_moe_layer *l, int batch) {
+    const size_t staged = staged_ws_bytes(l, batch, false);
+    if (batch < kGroupedMinBatch) return staged;
+    return std::max(staged, grouped_ws_base(fused_layout(l, false)) + grouped_ws_bytes(l, batch));
 }
 
 // The single-launch path (moe_fused.hip), in the regions `fl` places.

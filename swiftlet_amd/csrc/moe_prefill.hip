@@ -2066,6 +2066,17 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
 }
 
 }  // namespace
+
+size_t grouped_ws_bytes(const swq_moe_layer *l, int batch) {
+    return check_prefill_layer(l, batch) == SWQ_OK ? pf_layout(l, batch).total : 0;
+}
+
+int grouped_decode(const swq_moe_layer *layer, const void *x, int x_dtype, int batch, void *out, int out_dtype,
+                   int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes, int flags, hipStream_t stream) {
+    return prefill_impl(layer, x, x_dtype, batch, out, out_dtype, topk_ids, topk_weights, nullptr, ws, ws_bytes, flags,
+                        SWQ_PREFILL_ALL, stream);
+}
+
 }  // namespace swq
 
 using namespace swq;

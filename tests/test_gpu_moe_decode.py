@@ -6,6 +6,8 @@ logit gap exceeds 1e-3 (f32 summation-order noise of the router GEMV is
 ~1e-6 here); combine weights within 1e-5; layer output within 1e-3
 relative L2 of the f32 oracle (the observed error is ~1e-6)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -386,3 +388,48 @@ def test_f32_scales_equal_f16_scales(name, batch):
     torch.cuda.synchronize()
     assert a.workspace_error(wa, batch) == 0 and b.workspace_error(wb, batch) == 0
     assert torch.equal(ia, ib) and torch.equal(ka, kb) and torch.equal(oa, ob)
+
+
+@pytest.mark.parametrize("name,batch,x_dtype,grouped", [
+    ("qwen3.6-35b-a3b-q4", 5, "bf16", True), ("qwen3.6-35b-a3b-q4", 16, "f32", True),
+    ("qwen3.6-35b-a3b-q8", 6, "bf16", False), ("qwen3.6-35b-a3b-q8", 7, "bf16", True),
+    ("qwen3.6-35b-a3b-q8", 5, "f32", False), ("qwen3.6-35b-a3b-q8", 6, "f32", True)])
+def test_wide_batches_take_the_grouped_path(name, batch, x_dtype, grouped):
+    """On either side of the line between the three launches and the grouped path: the step equals
+    bit for bit the one that it should be (staged decode, prefill of the same tokens), through a
+    caller's workspace and through the static array, adding to out and writing bf16 too; and both
+    stay within 1e-5 relative L2 of each other (16 significant bits of h on either side: 2^-17
+    relative per element, averaged over the sums)."""
+    import torch
+    shape = synth.SHAPES[name]
+    gpu = moe.synth_layer(shape, helpers.SEED, 0)
+    xb = helpers.bf16_bits_to_torch(synth.activations_bf16(helpers.SEED + 300 + batch, batch, shape.hidden))
+    x = xb.float() * 1.1 if x_dtype == "f32" else xb
+    print(f"wide batch: {name} batch {batch} x {x_dtype} grouped {grouped}", flush=True)
+    ws = gpu.new_workspace(batch)
+    staged, i_s, w_s = gpu.decode(x, ws=ws, path="staged")
+    many, i_p, w_p = gpu.prefill(x)
+    out, ids, w = gpu.decode(x, ws=ws)
+    out2, ids2, w2 = gpu.decode(x, ws=ws)
+    acc = torch.ones_like(out)
+    gpu.decode(x, out=acc, ws=ws, accumulate=True)
+    narrow, _, _ = gpu.decode(x, out_dtype=torch.bfloat16, ws=ws)
+    torch.cuda.synchronize()
+    want, wi, ww = (many, i_p, w_p) if grouped else (staged, i_s, w_s)
+    assert torch.equal(out, want) and torch.equal(ids, wi) and torch.equal(w, ww)
+    assert torch.equal(out2, out) and torch.equal(ids2, ids) and torch.equal(w2, w)
+    assert torch.equal(acc, out + 1) and torch.equal(narrow, out.bfloat16())
+    assert torch.equal(i_s, i_p) and R.rel_l2(many.cpu().numpy(), staged.cpu().numpy()) < 1e-5
+    from swiftlet_amd import _lib
+    assert gpu.workspace_status(ws) == _lib.SWQ_OK
+    # the single launch on the same workspace afterwards
+    one, _, _ = gpu.decode(x[:1], ws=ws)
+    ref, _, _ = gpu.decode(x[:1], ws=gpu.new_workspace(1))
+    assert torch.equal(one, ref)
+    lib = _lib.load()
+    got = torch.empty_like(out)
+    code = {torch.float32: _lib.SWQ_F32, torch.bfloat16: _lib.SWQ_BF16}
+    _lib.check(lib.swq_moe_decode_noalloc(ctypes.byref(gpu._c), x.data_ptr(), code[x.dtype], batch, got.data_ptr(),
+                                          _lib.SWQ_F32, ids.data_ptr(), w.data_ptr(), 0, None), "noalloc")
+    torch.cuda.synchronize()
+    assert torch.equal(got, out) and torch.equal(ids, wi)
