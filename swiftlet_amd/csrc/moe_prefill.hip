@@ -51,7 +51,7 @@ constexpr int kLdsPitch = 72;    // bf16 per staged row: 64 + 8 (144 B rows, con
 constexpr int kMaxGroups = 64;   // inputs per row <= 4096
 constexpr int kXsPitch = kMaxGroups + 36;  // a K slice's bias term reads up to 31 groups past its first
 constexpr int kTileRows = 64;    // rows of a routed / shared tile
-constexpr int kRouterRows = 16;  // rows of a router tile
+constexpr int kRouterRows = 16;  // rows of a router tile, or twice that
 constexpr int kRouteWaves = 1;   // tokens per route workgroup, one wave each (512 workgroups at 512 tokens)
 constexpr int kXcds = 8;         // XCDs of the device: workgroup b runs on XCD b % 8
 
@@ -1320,6 +1320,7 @@ struct RouteArgs {
     int32_t *tok;             // [P + T]: token of each sorted row
     Tile *tiles;
     int32_t *n_tiles;
+    int32_t *counts;          // [kGroupSplit][E]: pf_count's
     int32_t T, E, K, H, norm, has_shared;
     int32_t tile_rows;        // most rows of a tile: kTileRows or kThinRows
     int32_t lslices;
@@ -1380,7 +1381,12 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 // second pass hands out the slots; the order of pairs within an expert does
 // not matter, every row is computed on its own).  The first kHeldIds * NT
 // ids are loaded at once and kept in registers for the second pass.
-template <int NT>
+//
+// SPLIT: one of gridDim.x workgroups, each with a share of the pairs, whose
+// counts per expert pf_count left in a.counts: every one scans the sums, its
+// slots start after those of the workgroups before it, and the first writes
+// the table.
+template <int NT, bool SPLIT>
 __device__ void group_pairs(const RouteArgs &a) {
     __shared__ int32_t s_cnt[kMaxExperts];  // counts, then the next free slot
     __shared__ int32_t s_wsum[2][NT / kWave];
@@ -1389,32 +1395,51 @@ __device__ void group_pairs(const RouteArgs &a) {
     constexpr int kHeldIds = 4096 / NT;  // every id of 512 tokens x top-8
     constexpr int kBatch = 8;  // ids per thread per pass past the held ones, all in flight at once
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const bool first = !SPLIT || blockIdx.x == 0;
     const int P = a.T * a.K, cap = a.tile_rows;
+    // this workgroup's pairs [pb, pe)
+    const int share = SPLIT ? (P + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x) : P;
+    const int pb = SPLIT ? min(static_cast<int>(blockIdx.x) * share, P) : 0, pe = SPLIT ? min(pb + share, P) : P;
     int held[kHeldIds];
 #pragma unroll
-    for (int u = 0; u < kHeldIds; ++u) held[u] = a.ids[min(tid + u * NT, P - 1)];
+    for (int u = 0; u < kHeldIds; ++u) held[u] = a.ids[min(pb + tid + u * NT, P - 1)];
     for (int e = tid; e < a.E; e += NT) s_cnt[e] = 0;
     for (int r = tid; r <= kTileRows; r += NT) s_rows[r] = 0;
     __syncthreads();
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int u = 0; u < kHeldIds; ++u)
-        if (tid + u * NT < P) atomicAdd(&s_cnt[held[u]], 1);
-    for (int p0 = tid + kHeldIds * NT; p0 < P; p0 += kBatch * NT) {
-        int e[kBatch];
+        for (int u = 0; u < kHeldIds; ++u)
+            if (tid + u * NT < P) atomicAdd(&s_cnt[held[u]], 1);
+        for (int p0 = tid + kHeldIds * NT; p0 < P; p0 += kBatch * NT) {
+            int e[kBatch];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) e[u] = a.ids[min(p0 + u * NT, P - 1)];
+            for (int u = 0; u < kBatch; ++u) e[u] = a.ids[min(p0 + u * NT, P - 1)];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-            if (p0 + u * NT < P) atomicAdd(&s_cnt[e[u]], 1);
+            for (int u = 0; u < kBatch; ++u)
+                if (p0 + u * NT < P) atomicAdd(&s_cnt[e[u]], 1);
+        }
     }
     __syncthreads();
     constexpr int EPT = kMaxExperts / NT;  // experts per thread
-    int cnt[EPT], tl[EPT];
+    int cnt[EPT], tl[EPT], before[EPT];  // before: the earlier workgroups' pairs of the expert
     int csum = 0, tsum = 0;
 #pragma unroll
     for (int i = 0; i < EPT; ++i) {
         const int e = tid * EPT + i;
-        cnt[i] = e < a.E ? s_cnt[e] : 0;
+        before[i] = 0;
+        if constexpr (SPLIT) {
+            cnt[i] = 0;
+            if (e < a.E) {
+#pragma unroll 8
+                for (int w = 0; w < static_cast<int>(gridDim.x); ++w) {
+                    const int c = a.counts[w * a.E + e];
+                    cnt[i] += c;
+                    before[i] += w < static_cast<int>(blockIdx.x) ? c : 0;
+                }
+            }
+        } else {
+            cnt[i] = e < a.E ? s_cnt[e] : 0;
+        }
         tl[i] = (cnt[i] + cap - 1) / cap;
         csum += cnt[i];
         tsum += tl[i];
@@ -1460,44 +1485,45 @@ __device__ void group_pairs(const RouteArgs &a) {
     for (int i = 0; i < EPT; ++i) {
         const int e = tid * EPT + i;
         if (e < a.E) {
-            s_cnt[e] = c0;  // each thread rewrites only its own experts
-            for (int q = 0; q < tl[i]; ++q) {
+            s_cnt[e] = c0 + before[i];  // each thread rewrites only its own experts
+            for (int q = 0; q < (first ? tl[i] : 0); ++q) {
                 const int rows = min(cap, cnt[i] - q * cap);
                 a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{e, c0 + q * cap, rows, 0};
             }
         }
         c0 += cnt[i];
     }
-    for (int q = tid; q < sh_tiles; q += NT) {
+    for (int q = tid; q < (first ? sh_tiles : 0); q += NT) {
         const int rows = min(cap, a.T - q * cap);
         a.tiles[atomicAdd(&s_rows[rows], 1)] = Tile{a.E, P + q * cap, rows, 0};
     }
-    if (tid == 0) *a.n_tiles = routed_tiles + sh_tiles;
+    if (first && tid == 0) *a.n_tiles = routed_tiles + sh_tiles;
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kHeldIds; ++u) {
-        const int p = tid + u * NT;
-        if (p < P) {
+        const int p = pb + tid + u * NT;
+        if (p < pe) {
             const int q = atomicAdd(&s_cnt[held[u]], 1);
             a.pos[p] = q;
             a.tok[q] = p / a.K;
         }
     }
-    for (int p0 = tid + kHeldIds * NT; p0 < P; p0 += kBatch * NT) {
+    for (int p0 = pb + tid + kHeldIds * NT; p0 < pe; p0 += kBatch * NT) {
         int e[kBatch];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) e[u] = a.ids[min(p0 + u * NT, P - 1)];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
             const int p = p0 + u * NT;
-            if (p >= P) continue;
+            if (p >= pe) continue;
             const int q = atomicAdd(&s_cnt[e[u]], 1);
             a.pos[p] = q;
             a.tok[q] = p / a.K;
         }
     }
     if (a.has_shared)
-        for (int t = tid; t < a.T; t += NT) a.tok[P + t] = t;
+        for (int t = (SPLIT ? static_cast<int>(blockIdx.x) * NT : 0) + tid; t < a.T; t += SPLIT ? NT * static_cast<int>(gridDim.x) : NT)
+            a.tok[P + t] = t;
 }
 
 // One token's routing on one wave: the logits of the lane's experts
@@ -1599,7 +1625,26 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void pf_route(const RouteArgs 
 // the kernel boundary orders the routing's stores before the grouping's
 // loads (an arrival count with a release per routing workgroup cost more).
 constexpr int kGroupThreads = 1024;
-__global__ __launch_bounds__(kGroupThreads) void pf_group(const RouteArgs a) { group_pairs<kGroupThreads>(a); }
+__global__ __launch_bounds__(kGroupThreads) void pf_group(const RouteArgs a) { group_pairs<kGroupThreads, false>(a); }
+
+// Many pairs: two launches of kGroupSplit workgroups, the counts per expert of
+// each share of the pairs, then the grouping of each share.  One workgroup
+// walks 32,768 pairs' LDS counters in 27 us (16,384 in 15), these two take
+// 4.6 + 8.3 (4.8 + 6.9); 8,192 pairs take it 9.6.
+constexpr int kGroupSplit = 32;
+constexpr int kGroupSplitPairs = 8192;  // from so many on
+constexpr int kCountThreads = 256;
+__global__ __launch_bounds__(kCountThreads) void pf_count(const RouteArgs a) {
+    __shared__ int32_t s_cnt[kMaxExperts];
+    const int P = a.T * a.K, share = (P + kGroupSplit - 1) / kGroupSplit;
+    const int pb = min(static_cast<int>(blockIdx.x) * share, P), pe = min(pb + share, P);
+    for (int e = threadIdx.x; e < a.E; e += kCountThreads) s_cnt[e] = 0;
+    __syncthreads();
+    for (int p = pb + threadIdx.x; p < pe; p += kCountThreads) atomicAdd(&s_cnt[a.ids[p]], 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < a.E; e += kCountThreads) a.counts[blockIdx.x * a.E + e] = s_cnt[e];
+}
+__global__ __launch_bounds__(kGroupThreads) void pf_group_split(const RouteArgs a) { group_pairs<kGroupThreads, true>(a); }
 
 // ---------------------------------------------------------------------------
 // combine
@@ -1673,8 +1718,16 @@ bool thin_tiles(const swq_moe_layer *l, int T) {
     return T <= kThinRows || static_cast<int64_t>(T) * l->top_k <= static_cast<int64_t>(kThinAvgRows) * l->num_experts;
 }
 
+// From kRouterWide tokens on the router's tiles have twice the rows, which halves the passes
+// over its codes; below, the smaller tiles are what fills the device.  us at 1,024 / 2,048 /
+// 4,096 tokens (256 experts, 2048 inputs, bf16 x): 16-token tiles 16.9 / 26.1 / 44.2, 32-token
+// ones 14.8 / 22.4 / 35.0 (64-token ones 15.2 / 19.4 / 31.8, but with f32 x 53 against 39 us at
+// 2,048 tokens of 512 experts; every slice in one workgroup, a single plane of logits for the
+// routing to read, 46 at 4,096 and nothing gained there).
+constexpr int kRouterWide = 1024;
+
 struct PfLayout {
-    size_t header, logits, sg, ids, wts, pos, tok, tiles, xs_x, xs_h, xa0, xa1, h_hi, h_lo, y, total;
+    size_t header, counts, logits, sg, ids, wts, pos, tok, tiles, xs_x, xs_h, xa0, xa1, h_hi, h_lo, y, total;
     int max_tiles, Ih, xs_ld_x, xs_ld_h, kslices;
 };
 
@@ -1694,6 +1747,7 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
                   (l->has_shared ? (T + cap - 1) / cap : 0);
     w.Ih = std::max(l->moe_intermediate, l->has_shared ? l->shared_intermediate : 0);
     w.header = take(256);  // [1] tile count
+    w.counts = P > kGroupSplitPairs ? take(static_cast<size_t>(kGroupSplit) * l->num_experts * 4) : 0;
     w.kslices = router_kslices(l->hidden);
     w.logits = take(static_cast<size_t>(w.kslices) * T * l->num_experts * 4);  // [slice][T][E] partial logits
     w.sg = take(static_cast<size_t>(T) * 4);
@@ -1934,9 +1988,15 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.pl0 = planes ? xa0 : nullptr;
         g.pl1 = planes && !bf16x ? xa1 : nullptr;
         g.pl_perm = perm_x ? 1 : 0;
-        const int blocks = gemm_blocks((T + kRouterRows - 1) / kRouterRows, g.nblk);
-        st = bf16x ? launch_gemm<kSrcBF16, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s)
-                   : launch_gemm<kSrcF32, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s);
+        const bool wide = T >= kRouterWide;
+        const int tile = wide ? 2 * kRouterRows : kRouterRows;
+        const int blocks = gemm_blocks((T + tile - 1) / tile, g.nblk);
+        if (!wide)
+            st = bf16x ? launch_gemm<kSrcBF16, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s)
+                       : launch_gemm<kSrcF32, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s);
+        else
+            st = bf16x ? launch_gemm<kSrcBF16, 2, kEpiRows, kSumStage>(layer->router, g, blocks, s)
+                       : launch_gemm<kSrcF32, 2, kEpiRows, kSumStage>(layer->router, g, blocks, s);
         if (st != SWQ_OK) return st;
     }
     // 2. routing and grouping
@@ -1968,7 +2028,14 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         if (bf16x) hipLaunchKernelGGL(pf_route<SWQ_BF16>, dim3(blocks), dim3(kRouteWaves * kWave), 0, s, r);
         else hipLaunchKernelGGL(pf_route<SWQ_F32>, dim3(blocks), dim3(kRouteWaves * kWave), 0, s, r);
         if ((st = launch_status()) != SWQ_OK) return st;
-        hipLaunchKernelGGL(pf_group, dim3(1), dim3(kGroupThreads), 0, s, r);
+        if (P > kGroupSplitPairs) {
+            r.counts = reinterpret_cast<int32_t *>(wsb + wl.counts);
+            hipLaunchKernelGGL(pf_count, dim3(kGroupSplit), dim3(kCountThreads), 0, s, r);
+            if ((st = launch_status()) != SWQ_OK) return st;
+            hipLaunchKernelGGL(pf_group_split, dim3(kGroupSplit), dim3(kGroupThreads), 0, s, r);
+        } else {
+            hipLaunchKernelGGL(pf_group, dim3(1), dim3(kGroupThreads), 0, s, r);
+        }
         if ((st = launch_status()) != SWQ_OK) return st;
     }
     // 3. gate/up + SwiGLU over the tiles

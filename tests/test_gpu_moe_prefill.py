@@ -302,3 +302,28 @@ def test_few_tokens_equal_many(H, I, Is, bits, x_dtype, f32_scales):
         out, ids, w = gpu.prefill(x[:T].contiguous())
         torch.cuda.synchronize()
         assert torch.equal(ids, want_ids[:T]) and torch.equal(w, want_w[:T]) and torch.equal(out, want[:T]), T
+
+
+@pytest.mark.parametrize("E,K,T,x_dtype", [(60, 9, 911, "bf16"), (256, 8, 1024, "f32"), (256, 8, 1025, "bf16"),
+                                           (513, 5, 2049, "bf16"), (256, 8, 3073, "bf16"), (520, 16, 1311, "f32")])
+def test_many_tokens_equal_few(E, K, T, x_dtype):
+    """The router's 32-token tiles (from 1,024 tokens) and the grouping over several workgroups
+    (from 8,193 pairs): routing and outputs of every token equal, bit for bit, those of calls of at most 500 of the
+    tokens, which take none of them.  The expert loads are skewed; the pairs of the last share and
+    the last tiles are ragged."""
+    import torch
+    shape = synth.MoEShape("many", 512, E, K, 128, 128, expert_bits=4, router_bits=8, group=64, norm_topk_prob=True)
+    gpu = moe.synth_layer(shape, 5000 + E, 0)
+    bias = torch.from_numpy(synth.zipf_logit_bias(ZIPF_SEED, E)).cuda()
+    x, _ = _x(31 + T, T, 512)
+    if x_dtype == "f32":
+        x = x.float() * 1.1
+    print(f"many tokens: E {E} K {K} T {T} x {x_dtype}", flush=True)
+    ws = gpu.new_prefill_workspace(T)
+    for _ in range(2):
+        out, ids, w = gpu.prefill(x, ws=ws, logit_bias=bias)
+        for lo in range(0, T, 500):
+            o, i, ww = gpu.prefill(x[lo:lo + 500].contiguous(), logit_bias=bias)
+            torch.cuda.synchronize()
+            n = o.shape[0]
+            assert torch.equal(i, ids[lo:lo + n]) and torch.equal(ww, w[lo:lo + n]) and torch.equal(o, out[lo:lo + n]), lo
