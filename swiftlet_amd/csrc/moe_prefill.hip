@@ -1862,18 +1862,20 @@ int launch_gemm(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream
 // gate/up (bf16 x): 8 waves (256 down or 128 gate/up columns per workgroup:
 // the tile's activation rows are shared by twice the columns), two
 // workgroups in a CU's 160 KB of LDS.  4-bit gate/up with bf16 x: 4 waves
-// (64 columns, 49 KB), three workgroups per CU: twice the workgroups, which
+// (64 columns, 38 KB), four workgroups per CU: twice the workgroups, which
 // spreads the last, partly filled round of tiles over more CUs (gate/up
-// 113 -> 108.5 us on the 512-token chunk; down at 4 waves fits only two
-// per CU and loses, 80 -> 87 us).  8-bit codes with two activation planes:
-// 4 waves.
+// 113 -> 108.5 us on the 512-token chunk; down at 4 waves loses, 74 -> 79 us
+// there, 261 -> 280 at 4,096 tokens).  8-bit codes with two activation planes:
+// 4 waves.  Activation rings are two groups deep: four workgroups per CU, 16
+// waves, cover the waits better than a third group in the LDS of three does
+// (4-bit gate/up, bf16 x: 106.7 -> 97.8 us at 512 tokens, 322 -> 302 at 4,096;
+// five, with the group sums read at the end instead of held in LDS, spill).
 int dma_waves(int bits, int npl) { return (bits == 8 && npl == 2) || (bits == 4 && npl == 1) ? 4 : 8; }
 
 template <int BITS, int NPL, int EPI>
 void launch_dma_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
     constexpr int W = (BITS == 8 && NPL == 2) || (BITS == 4 && NPL == 1) ? 4 : 8;
-    constexpr int DA = BITS == 4 && NPL == 1 ? 3 : 2;
-    constexpr int DB = DA + 1;
+    constexpr int DA = 2, DB = DA + 1;
     const dim3 th(64 * W);
     if (stype == SWQ_F16)
         hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F16, NPL, EPI, DA, DB, W>), dim3(blocks), th, 0, s, a);
