@@ -399,14 +399,14 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine(const AttnArgs a
 #pragma unroll
     for (int u = 0; u < U; ++u)
         v[u] = *reinterpret_cast<const float4 *>(src + static_cast<int64_t>(min(s0 + u * SPR, a.splits - 1)) * HD);
-    float M = wave_max(ms);
+    float M = wave_max_all(ms);
     if (lane == 0) s_red[0][wave] = M;
     lds_barrier();
 #pragma unroll
     for (int w = 0; w < kCombineWaves; ++w) M = fmaxf(M, s_red[0][w]);
     const float wt = mine ? expf(ms - finite_max(M)) : 0.f;
     if (tid < a.splits) s_w[tid] = wt;
-    const float lw = wave_sum(wt * ls);
+    const float lw = wave_sum_all(wt * ls);
     if (lane == 0) s_red[1][wave] = lw;
     lds_barrier();
     float acc[4] = {0.f, 0.f, 0.f, 0.f};

@@ -40,6 +40,18 @@ __device__ __forceinline__ float wave_sum_all(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(segment_reduce(v, 6)), 63));
 }
 
+// Maximum over the wave, returned to every lane (fmaxf: a NaN loses to a number).
+__device__ __forceinline__ float wave_max_all(float v) {
+    v = fmaxf(v, dpp<0xB1, 0xF, true>(v));   // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp<0x4E, 0xF, true>(v));   // quad_perm [2,3,0,1]
+    v = fmaxf(v, dpp<0x141, 0xF, true>(v));  // row_half_mirror
+    v = fmaxf(v, dpp<0x140, 0xF, true>(v));  // row_mirror
+    const int i = __float_as_int(v);
+    const float r0 = __int_as_float(__builtin_amdgcn_readlane(i, 0)), r1 = __int_as_float(__builtin_amdgcn_readlane(i, 16));
+    const float r2 = __int_as_float(__builtin_amdgcn_readlane(i, 32)), r3 = __int_as_float(__builtin_amdgcn_readlane(i, 48));
+    return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
+}
+
 // routing: top-k of the logits in LDS, one wave
 
 // Lane l holds experts l*M .. l*M+M-1, sorted by (logit desc, id asc); each
