@@ -55,6 +55,7 @@
 #include "route.hpp"
 #include "tile.hpp"
 
+#include <type_traits>
 #include <utility>
 
 // Phase stamps for timing studies: SWQ_FUSED_TRACE builds record
@@ -567,41 +568,49 @@ __global__ __launch_bounds__(kFusedThreads) __attribute__((amdgpu_waves_per_eu(k
         // s_x = (h_in + res_in) * (scale * w) (QwenCPUModel.rmsNorm and the
         // residual add before it, QwenCPUModel.swift:47-59, :276-277); one
         // round trip, indices clamped, values past H masked
-        constexpr int kPer = kPrenormMaxHidden / kFusedThreads;
         const bool has_r = a.res_in != nullptr, wf32 = a.norm_dtype == SWQ_F32;
         const float *rp = has_r ? a.res_in : a.h_in;
-        float hr[kPer], rr[kPer];
-        uint32_t wr[kPer];
+        // KPER elements per thread, loads unconditional (clamped): as few as hidden sizes up to
+        // 2048 need, since every wave of the CU issues them ahead of its first weights (48 loads
+        // per thread for any size up to 8192 took the step 15.25 us, 12 take it 14.7)
+        auto prenorm = [&](auto KPER) {
+            constexpr int kPer = KPER();
+            float hr[kPer], rr[kPer];
+            uint32_t wr[kPer];
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int ic = min(static_cast<int>(threadIdx.x) + k * kFusedThreads, a.H - 1);
-            hr[k] = a.h_in[ic];
-            rr[k] = rp[ic];
-            wr[k] = wf32 ? static_cast<const uint32_t *>(a.norm_w)[ic] : static_cast<const uint16_t *>(a.norm_w)[ic];
-        }
-        float v[kPer], wv[kPer];
-        float ss = 0.f;
+            for (int k = 0; k < kPer; ++k) {
+                const int ic = min(static_cast<int>(threadIdx.x) + k * kFusedThreads, a.H - 1);
+                hr[k] = a.h_in[ic];
+                rr[k] = rp[ic];
+                wr[k] = wf32 ? static_cast<const uint32_t *>(a.norm_w)[ic] : static_cast<const uint16_t *>(a.norm_w)[ic];
+            }
+            float v[kPer], wv[kPer];
+            float ss = 0.f;
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const bool valid = static_cast<int>(threadIdx.x) + k * kFusedThreads < a.H;
-            v[k] = valid ? (has_r ? hr[k] + rr[k] : hr[k]) : 0.f;
-            wv[k] = wf32 ? __uint_as_float(wr[k])
-                         : (a.norm_dtype == SWQ_BF16 ? bf16_to_f32(static_cast<uint16_t>(wr[k]))
-                                                     : f16_to_f32(static_cast<uint16_t>(wr[k])));
-            ss += v[k] * v[k];
-        }
-        ss = wave_sum(ss);
-        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = ss;
-        __syncthreads();
-        float tot = 0.f;
+            for (int k = 0; k < kPer; ++k) {
+                const bool valid = static_cast<int>(threadIdx.x) + k * kFusedThreads < a.H;
+                v[k] = valid ? (has_r ? hr[k] + rr[k] : hr[k]) : 0.f;
+                wv[k] = wf32 ? __uint_as_float(wr[k])
+                             : (a.norm_dtype == SWQ_BF16 ? bf16_to_f32(static_cast<uint16_t>(wr[k]))
+                                                         : f16_to_f32(static_cast<uint16_t>(wr[k])));
+                ss += v[k] * v[k];
+            }
+            ss = wave_sum(ss);
+            if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = ss;
+            lds_barrier();
+            float tot = 0.f;
 #pragma unroll
-        for (int i = 0; i < kFusedWaves; ++i) tot += s_red[i];
-        const float sc = 1.0f / __fsqrt_rn(tot / static_cast<float>(a.H) + a.norm_eps);
+            for (int i = 0; i < kFusedWaves; ++i) tot += s_red[i];
+            const float sc = 1.0f / __fsqrt_rn(tot / static_cast<float>(a.H) + a.norm_eps);
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int i = threadIdx.x + k * kFusedThreads;
-            if (i < a.H) s_x[i] = v[k] * (sc * wv[k]);
-        }
+            for (int k = 0; k < kPer; ++k) {
+                const int i = threadIdx.x + k * kFusedThreads;
+                if (i < a.H) s_x[i] = v[k] * (sc * wv[k]);
+            }
+        };
+        constexpr int kFew = 2048 / kFusedThreads;
+        if (a.H <= 2048) prenorm(std::integral_constant<int, kFew>{});
+        else prenorm(std::integral_constant<int, kPrenormMaxHidden / kFusedThreads>{});
         x = s_x;
     }
     __syncthreads();
