@@ -461,8 +461,8 @@ int swq_moe_workspace_status(void *ws, size_t ws_bytes, int clear, void *stream)
  *   2. top-k per token, the distinct experts, their gate/up SwiGLU rows for
  *      all their tokens, indexed by the device-resident ids;
  *   3. down projections + weighted combine + sigmoid-gated shared expert;
- * or, from five tokens on where the experts are large enough, as
- * swq_moe_prefill's launches (the pairs sorted by expert, matrix cores), if
+ * or, from five tokens on with bf16 x and 4-bit experts that are large enough,
+ * as swq_moe_prefill's launches (the pairs sorted by expert, matrix cores), if
  * the prefill takes the layer, out is 16-byte aligned and the workspace holds
  * swq_moe_decode_workspace_bytes(layer, batch).
  * x: [batch, hidden] of x_dtype (SWQ_F32 / SWQ_BF16).  out: [batch, hidden]

@@ -161,27 +161,30 @@ int grouped_decode(const swq_moe_layer *layer, const void *x, int x_dtype, int b
                    int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes, int flags, hipStream_t stream);
 inline size_t grouped_ws_base(const FusedLayout &f) { return align256(f.total); }
 
-// Where the grouped path is the faster one: the three launches' time goes with
-// the codes that every (token, pick) pair multiplies, the grouped path's with
-// the distinct experts' bytes on top of its six launches.  us for three
-// launches / grouped, 256 experts top-8 (3.1 M codes a pair):
-//   batch             5      6      7      8      11      16
-//   4-bit, bf16 x   58/55  65/55  72/58  78/59  103/68  135/79
-//   4-bit, f32 x    65/57  74/58  82/60  90/61  116/74  157/86
-//   8-bit, bf16 x   54/62  60/63  68/67  71/70   91/82  121/104
-//   8-bit, f32 x    59/64  67/64  75/68  81/72  106/86  141/107
-// and 512 experts top-10, 4-bit, bf16 x: 71/61 at 5, 170/98 at 16.
+// Where the grouped path is taken: bf16 activations and 4-bit experts, for which
+// it is as exact as the three launches (x exact, h in 16 significant bits on
+// either side: 3.5e-6 relative against 64 bits there, 2.8e-6 grouped), and where
+// it is the faster one: the three launches' time goes with the codes that every
+// (token, pick) pair multiplies, the grouped path's with the distinct experts'
+// bytes on top of its six launches.  us for three launches / grouped:
+//   batch                          5      6      7      8      11      16
+//   256 experts top-8 (3.1 M
+//   codes a pair)                58/55  65/55  72/58  78/59  103/68  135/79
+//   512 experts top-10           71/61  79/63  89/67  95/71  126/84  170/98
+// f32 activations and 8-bit experts stay with the three launches, which keep x
+// and h in 32 bits there (5e-7 relative; the grouped path splits both to 16
+// significant bits, 5.6e-6), though it would be the faster one at 16 tokens
+// (8-bit 121/104).
 constexpr int kGroupedMinBatch = 5;
 inline bool grouped_pays(const swq_moe_layer *l, int x_dtype, int batch) {
-    const double codes = 3.0 * batch * l->top_k * l->hidden * l->moe_intermediate;
-    return batch >= kGroupedMinBatch && codes >= (l->gate.bits == 4 ? 120e6 : (x_dtype == SWQ_F32 ? 150e6 : 175e6));
+    if (x_dtype != SWQ_BF16 || l->gate.bits != 4 || l->down.bits != 4) return false;
+    return batch >= kGroupedMinBatch && 3.0 * batch * l->top_k * l->hidden * l->moe_intermediate >= 120e6;
 }
 
-// Bytes of the whole decode workspace for `batch` tokens: whatever batch up to
-// that and whatever activations the calls bring.
+// Bytes of the whole decode workspace for up to `batch` tokens of either type.
 inline size_t decode_ws_bytes(const swq_moe_layer *l, int batch) {
     const size_t staged = staged_ws_bytes(l, batch, false);
-    if (batch < kGroupedMinBatch) return staged;
+    if (!grouped_pays(l, SWQ_BF16, batch)) return staged;
     return std::max(staged, grouped_ws_base(fused_layout(l, false)) + grouped_ws_bytes(l, batch));
 }
 

@@ -391,9 +391,9 @@ def test_f32_scales_equal_f16_scales(name, batch):
 
 
 @pytest.mark.parametrize("name,batch,x_dtype,grouped", [
-    ("qwen3.6-35b-a3b-q4", 5, "bf16", True), ("qwen3.6-35b-a3b-q4", 16, "f32", True),
-    ("qwen3.6-35b-a3b-q8", 6, "bf16", False), ("qwen3.6-35b-a3b-q8", 7, "bf16", True),
-    ("qwen3.6-35b-a3b-q8", 5, "f32", False), ("qwen3.6-35b-a3b-q8", 6, "f32", True)])
+    ("qwen3.6-35b-a3b-q4", 5, "bf16", True), ("qwen3.6-35b-a3b-q4", 16, "bf16", True),
+    ("qwen3.6-35b-a3b-q4", 16, "f32", False), ("qwen3.6-35b-a3b-q8", 16, "bf16", False),
+    ("qwen3-next-80b-a3b-q4", 7, "bf16", True)])
 def test_wide_batches_take_the_grouped_path(name, batch, x_dtype, grouped):
     """On either side of the line between the three launches and the grouped path: the step equals
     bit for bit the one that it should be (staged decode, prefill of the same tokens), through a
