@@ -161,23 +161,31 @@ int grouped_decode(const swq_moe_layer *layer, const void *x, int x_dtype, int b
                    int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes, int flags, hipStream_t stream);
 inline size_t grouped_ws_base(const FusedLayout &f) { return align256(f.total); }
 
-// Where the grouped path is taken: bf16 activations and 4-bit experts, for which
-// it is as exact as the three launches (x exact, h in 16 significant bits on
-// either side: 3.5e-6 relative against 64 bits there, 2.8e-6 grouped), and where
-// it is the faster one: the three launches' time goes with the codes that every
-// (token, pick) pair multiplies, the grouped path's with the distinct experts'
-// bytes on top of its six launches.  us for three launches / grouped:
+// Where the grouped path is taken: bf16 activations, 4-bit experts and 2-byte
+// scales, for which it is as exact as the three launches (x exact, h in 16
+// significant bits on either side: 3.5e-6 relative against 64 bits there, 2.8e-6
+// grouped), and where it is the faster one: the three launches' time goes with
+// the codes that every (token, pick) pair multiplies, the grouped path's with the
+// distinct experts' bytes on top of its six launches.  us for three launches /
+// grouped:
 //   batch                          5      6      7      8      11      16
 //   256 experts top-8 (3.1 M
 //   codes a pair)                58/55  65/55  72/58  78/59  103/68  135/79
 //   512 experts top-10           71/61  79/63  89/67  95/71  126/84  170/98
-// f32 activations and 8-bit experts stay with the three launches, which keep x
-// and h in 32 bits there (5e-7 relative; the grouped path splits both to 16
-// significant bits, 5.6e-6), though it would be the faster one at 16 tokens
-// (8-bit 121/104).
+// Its bias term takes b - 16 s as two bf16 (16 significant bits): whole for f16
+// and bf16 scales, whose sum fits them where b is within a factor of 32 (f16) or
+// 256 (bf16) of 16 s, as quantisers place it; not for f32 ones (1e-5 of one
+// product).  f32 scales on any matrix, f32 activations and 8-bit experts stay with
+// the three launches, which keep scales, x and h in 32 bits there (5e-7 relative;
+// the grouped path splits x and h to 16 significant bits, 5.6e-6), though it would
+// be the faster one at 16 tokens (8-bit 121/104, f32 scales 133/119; at 5 tokens
+// f32 scales 56/69).
 constexpr int kGroupedMinBatch = 5;
 inline bool grouped_pays(const swq_moe_layer *l, int x_dtype, int batch) {
     if (x_dtype != SWQ_BF16 || l->gate.bits != 4 || l->down.bits != 4) return false;
+    auto f32 = [](const swq_qlinear &m) { return m.scales_type == SWQ_F32; };
+    if (f32(l->router) || f32(l->gate) || f32(l->up) || f32(l->down)) return false;
+    if (l->has_shared && (f32(l->shared_gate) || f32(l->shared_up) || f32(l->shared_down))) return false;
     return batch >= kGroupedMinBatch && 3.0 * batch * l->top_k * l->hidden * l->moe_intermediate >= 120e6;
 }
 

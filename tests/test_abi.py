@@ -83,6 +83,23 @@ def test_workspace_query(lib):
     assert lib.swq_moe_decode_workspace_bytes(ctypes.byref(L), 17) == 0  # above SWQ_MAX_BATCH
 
 
+EXPERTS = ("gate", "up", "down", "shared_gate", "shared_up", "shared_down")
+
+
+@pytest.mark.parametrize("wide", [("router",), EXPERTS, ("router",) + EXPERTS], ids=["router", "experts", "all"])
+def test_f32_scales_keep_the_three_launches(lib, wide):
+    """A wide batch is regrouped by expert only where every scale has two bytes (the regrouped
+    contraction holds b - 16 s in 16 significant bits): with f32 scales the workspace is that of
+    the three launches, as it is for 8-bit experts."""
+    L = layer()
+    staged = lib.swq_moe_decode_workspace_bytes(ctypes.byref(layer(bits=8)), 8)
+    assert lib.swq_moe_decode_workspace_bytes(ctypes.byref(L), 8) > staged
+    for matrix in wide:
+        getattr(L, matrix).scales_type = _lib.SWQ_F32
+        getattr(L, matrix).expert_stride_sb *= 2
+    assert lib.swq_moe_decode_workspace_bytes(ctypes.byref(L), 8) == staged
+
+
 def decode(lib, L, batch=1, ws_bytes=None, x=FAKE, x_dtype=_lib.SWQ_BF16, out_dtype=_lib.SWQ_F32, flags=0, ws=FAKE):
     if ws_bytes is None:
         ws_bytes = max(lib.swq_moe_decode_workspace_bytes(ctypes.byref(L), batch), 1 << 20)

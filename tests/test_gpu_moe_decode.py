@@ -433,3 +433,50 @@ def test_wide_batches_take_the_grouped_path(name, batch, x_dtype, grouped):
                                           _lib.SWQ_F32, ids.data_ptr(), w.data_ptr(), 0, None), "noalloc")
     torch.cuda.synchronize()
     assert torch.equal(got, out) and torch.equal(ids, wi)
+
+
+def _dense64(lin, e=0):
+    """Expert e of a 4- or 8-bit GPULinear in 64 bits, on the device."""
+    import torch
+    per = 32 // lin.bits
+    words = lin.w.view(torch.int32)[e * lin.expert_stride_w // 4:][:lin.out_dim * lin.in_dim // per].long()
+    codes = (words.unsqueeze(1) >> (lin.bits * torch.arange(per, device=words.device))) & ((1 << lin.bits) - 1)
+    n = lin.out_dim * lin.in_dim // lin.group_size
+    s, b = (t.view(torch.float32)[e * lin.expert_stride_sb // 4:][:n].double().unsqueeze(1) for t in (lin.scales, lin.biases))
+    return (codes.reshape(n, lin.group_size) * s + b).reshape(lin.out_dim, lin.in_dim)
+
+
+@pytest.mark.parametrize("name,batch", [("qwen3.6-35b-a3b-q4", 8), ("qwen3-next-80b-a3b-q4", 5)])
+def test_wide_batch_of_f32_scales(name, batch):
+    """Scales and biases that need all of their 32 bits, in a batch wide enough for the grouped
+    path with 2-byte ones: the three launches' bits, and within 1e-5 of 64 bits (the dot products
+    split h to 16 significant bits, 3.5e-6; a bias term in 16 bits would add 1e-5 per product)."""
+    import torch
+    shape = synth.SHAPES[name]
+    gpu = helpers.widen_layer(moe.synth_layer(shape, helpers.SEED, 0))
+    g = torch.Generator(device="cuda").manual_seed(7)
+    mats = [gpu.router, gpu.gate, gpu.up, gpu.down, gpu.shared_gate, gpu.shared_up, gpu.shared_down]
+    for m in mats:
+        for t in (m.scales, m.biases):
+            f = t.view(torch.float32)
+            f.mul_(1 + 0.01 * torch.rand(f.shape, generator=g, device="cuda"))
+    x = helpers.bf16_bits_to_torch(synth.activations_bf16(helpers.SEED + 17, batch, shape.hidden))
+    print(f"f32 scales: {name} batch {batch}", flush=True)
+    ws = gpu.new_workspace(batch)
+    staged, i_s, w_s = gpu.decode(x, ws=ws, path="staged")
+    out, ids, w = gpu.decode(x, ws=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, staged) and torch.equal(ids, i_s) and torch.equal(w, w_s)
+    xd = x.double()
+    probs = (xd @ _dense64(gpu.router).t()).softmax(1)
+    top = probs.gather(1, ids.long())
+    top = top / top.sum(1, keepdim=True)
+    ffn = lambda v, gm, um, dm: dm @ (torch.nn.functional.silu(gm @ v) * (um @ v))  # noqa: E731
+    seg = gpu.shared_expert_gate
+    want = torch.stack([sum(top[t, k] * ffn(xd[t], *(_dense64(m, int(ids[t, k])) for m in mats[1:4]))
+                            for k in range(shape.top_k)) for t in range(batch)])
+    gate = torch.sigmoid(xd @ _dense64(seg).t())
+    want += gate * torch.stack([ffn(xd[t], *(_dense64(m) for m in mats[4:])) for t in range(batch)])
+    err = R.rel_l2(out.double().cpu().numpy(), want.cpu().numpy())
+    print(f"  rel L2 {err:.2e} of 64 bits", flush=True)
+    assert err < 1e-5, err
