@@ -11,7 +11,7 @@ import ctypes
 
 from . import _lib
 from ._lib import AttentionLayer, check
-from .engine import DescArray, GPULinear, HipEngine, _norm_arg, _stream_handle, _torch
+from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch
 
 
 class AttentionGPU:
@@ -77,6 +77,9 @@ class AttentionGPU:
         """x [H_model] f32 -> the block's output: q/k/v_proj in one launch
         (with norm_weight, x is the un-normalised hidden state and the input
         RMSNorm runs inside that launch), the step, o_proj."""
+        if _elsewhere(stream):
+            with _torch().cuda.stream(stream):
+                return self.forward_token(engine, x, cache, ws, position, norm_weight, eps)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         pq, pk, pv = self.projections
         projs = self._projs.of((pq, pk, pv))

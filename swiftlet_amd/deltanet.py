@@ -10,7 +10,7 @@ import ctypes
 
 from . import _lib
 from ._lib import SWQ_DELTA_INTERLEAVED, SWQ_DELTA_SPLIT, DeltaNetLayer, check
-from .engine import DescArray, GPULinear, HipEngine, _norm_arg, _stream_handle, _torch
+from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch
 
 
 class DeltaNetGPU:
@@ -82,6 +82,9 @@ class DeltaNetGPU:
         """x [H] f32 -> the block's output [H]: the input projections in one
         launch (with norm_weight, x is the un-normalised hidden state and the
         input RMSNorm runs inside that launch), the step, out_proj."""
+        if _elsewhere(stream):
+            with _torch().cuda.stream(stream):
+                return self.forward_token(engine, x, state, position, norm_weight, eps)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         scratch = empty(self._scratch, dtype=f32, device=dev)
         r = empty(self.out_proj.out_dim, dtype=f32, device=dev)

@@ -35,6 +35,13 @@ def _stream_handle(stream) -> int:
     return _torch()._C._cuda_getCurrentRawStream(cuda.current_device())
 
 
+def _elsewhere(stream) -> bool:
+    """Whether `stream` is another than the current one: what a call allocates for itself and lets
+    go on return has then to come from that stream's memory, or the current stream may be handed
+    it while the call's work still runs."""
+    return stream is not None and stream != _torch().cuda.current_stream()
+
+
 def _norm_arg(weight):
     """(dtype code, address) of a norm weight, or those of none."""
     if weight is None:
@@ -233,7 +240,7 @@ class HipEngine:
         torch = _torch()
         dev = logits.device
         vocab = logits.numel()
-        if stream is not None and stream != torch.cuda.current_stream():
+        if _elsewhere(stream):
             with torch.cuda.stream(stream):
                 return self.sample(logits, temperature, top_k, top_p, presence, frequency, seen, banned, u, ws)
         if ws is None:
