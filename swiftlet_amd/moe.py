@@ -16,7 +16,7 @@ import numpy as np
 
 from . import _lib, synth
 from ._lib import SWQ_BF16, SWQ_F16, SWQ_F32, MoELayer, QLinear, check
-from .engine import GPULinear, _stream_handle, _torch
+from .engine import GPULinear, _elsewhere, _stream_handle, _torch
 
 
 def _empty_linear() -> QLinear:
@@ -160,6 +160,9 @@ class MoELayerGPU:
 
     def new_prefill_workspace(self, tokens: int, stream=None):
         torch = _torch()
+        if _elsewhere(stream):
+            with torch.cuda.stream(stream):
+                return self.new_prefill_workspace(tokens)
         n = self.prefill_workspace_bytes(tokens)
         ws = torch.empty(n, dtype=torch.uint8, device=self.router.w.device)
         check(self.lib.swq_moe_workspace_init(ws.data_ptr(), n, _stream_handle(stream)), "workspace_init")

@@ -9,13 +9,13 @@ import types
 
 import pytest
 
-from swiftlet_amd import attention, deltanet, engine
+from swiftlet_amd import attention, deltanet, engine, moe
 
 
 class FakeTorch:
     """empty() and the current stream of torch; `log` holds the stream of each allocation."""
 
-    float32 = "f32"
+    float32, bfloat16, int32, uint8 = "f32", "bf16", "i32", "u8"
 
     def __init__(self):
         self.current, self.log = types.SimpleNamespace(cuda_stream="default"), []
@@ -35,16 +35,16 @@ class FakeTorch:
 
 
 class FakeLib:
-    """Every entry returns success; `streams` holds the last argument of the token calls."""
+    """Every entry returns success; `streams` holds the last argument of the token and prefill calls."""
 
     def __init__(self):
         self.streams = []
 
     def __getattr__(self, name):
         def call(*args):
-            if name.endswith("_token"):
+            if name.endswith(("_token", "_prefill")):
                 self.streams.append(args[-1])
-            return 64 if name.endswith("_floats") else 0
+            return 64 if name.endswith(("_floats", "_bytes")) else 0
         return call
 
 
@@ -80,6 +80,22 @@ def test_token_scratch_is_allocated_on_the_given_stream(kind, monkeypatch):
     call(types.SimpleNamespace(cuda_stream="side"))
     assert fake.log == ["default"] * 2 + ["side"] * 2 and blk.lib.streams == ["default", "side"]
     assert fake.current.cuda_stream == "default"
+
+
+def test_prefill_workspace_is_allocated_on_the_given_stream(monkeypatch):
+    """A prefill without a workspace makes one and lets go of it on return."""
+    fake = FakeTorch()
+    for m in (engine, moe):
+        monkeypatch.setattr(m, "_torch", lambda: fake)
+    layer = moe.MoELayerGPU.__new__(moe.MoELayerGPU)
+    layer._c, layer.lib, layer.router, layer.hidden, layer.top_k = moe.MoELayer(), FakeLib(), _lin(), 64, 2
+    layer.router.w.device = "cuda"
+    buf = types.SimpleNamespace(data_ptr=lambda: 0x3000, device="cuda", dtype="f32", shape=(1, 64), dim=lambda: 2)
+    given = dict(out=buf, topk_ids=buf, topk_weights=buf)
+    layer.prefill(buf, **given)
+    assert fake.log == ["default"] and layer.lib.streams == ["default"]
+    layer.prefill(buf, stream=types.SimpleNamespace(cuda_stream="side"), **given)
+    assert fake.log == ["default", "side"] and layer.lib.streams == ["default", "side"]
 
 
 @pytest.mark.gpu
