@@ -510,10 +510,10 @@ extern "C" size_t swq_attention_workspace_bytes(const swq_attention_layer *l) {
     return static_cast<size_t>(l->num_heads) * splits * (l->head_dim + 2) * sizeof(float);
 }
 
-extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_proj, const float *k_proj,
-                                  const float *v_proj, void *cache, size_t cache_bytes, int64_t position,
-                                  float *out, void *ws, size_t ws_bytes, void *stream) {
-    int st = check_layer(l);
+static int check_step(const swq_attention_layer *l, const float *q_proj, const float *k_proj, const float *v_proj,
+                      const void *cache, size_t cache_bytes, int64_t position, const float *out, const void *ws,
+                      size_t ws_bytes) {
+    const int st = check_layer(l);
     if (st != SWQ_OK) return st;
     if (!q_proj || !k_proj || !v_proj || !cache || !out || position < 0) return SWQ_ERR_INVALID_ARGUMENT;
     if (position >= l->max_positions) return SWQ_ERR_LIMIT;
@@ -521,6 +521,14 @@ extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_p
     if (!ws || ws_bytes < swq_attention_workspace_bytes(l)) return SWQ_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(cache) % 256 != 0 || reinterpret_cast<uintptr_t>(ws) % 256 != 0)
         return SWQ_ERR_MISALIGNED;
+    return SWQ_OK;
+}
+
+extern "C" int swq_attention_step(const swq_attention_layer *l, const float *q_proj, const float *k_proj,
+                                  const float *v_proj, void *cache, size_t cache_bytes, int64_t position,
+                                  float *out, void *ws, size_t ws_bytes, void *stream) {
+    const int st = check_step(l, q_proj, k_proj, v_proj, cache, cache_bytes, position, out, ws, ws_bytes);
+    if (st != SWQ_OK) return st;
     AttnArgs a{};
     a.q_proj = q_proj;
     a.k_proj = k_proj;
@@ -588,6 +596,11 @@ extern "C" int swq_attention_token(const swq_attention_layer *l, const swq_qline
     float *q = scratch, *k = q + pad_floats(projections[0].out_dim), *v = k + pad_floats(projections[1].out_dim);
     float *y = v + pad_floats(projections[2].out_dim);
     float *ys[3] = {q, k, v};
+    // every check before the first launch: an error leaves the cache as it was
+    st = check_gemv_multi(projections, 3, ys, x, norm_weight, norm_dtype, norm_eps);
+    if (st == SWQ_OK) st = check_step(l, q, k, v, cache, cache_bytes, position, y, ws, ws_bytes);
+    if (st == SWQ_OK) st = check_gemv(o_proj, y, out);
+    if (st != SWQ_OK) return st;
     st = swq_encode_gemv_multi(projections, 3, ys, x, norm_weight, norm_dtype, norm_eps, stream);
     if (st == SWQ_OK) st = swq_attention_step(l, q, k, v, cache, cache_bytes, position, y, ws, ws_bytes, stream);
     if (st == SWQ_OK) st = swq_encode_gemv(o_proj, 0, 0, 0, 0, y, 0, out, 0, stream);

@@ -259,15 +259,22 @@ extern "C" size_t swq_deltanet_state_bytes(const swq_deltanet_layer *l) {
            static_cast<size_t>(l->num_value_heads) * l->value_head_dim * l->key_head_dim * sizeof(float);
 }
 
-extern "C" int swq_deltanet_step(const swq_deltanet_layer *l, const float *qkvz, const float *ba, void *state,
-                                 size_t state_bytes, int64_t position, float *out, void *stream) {
-    int st = check_layer(l);
+static int check_step(const swq_deltanet_layer *l, const float *qkvz, const float *ba, const void *state,
+                      size_t state_bytes, int64_t position, const float *out) {
+    const int st = check_layer(l);
     if (st != SWQ_OK) return st;
     if (!qkvz || !ba || !state || !out || position < 0) return SWQ_ERR_INVALID_ARGUMENT;
     if (state_bytes < swq_deltanet_state_bytes(l)) return SWQ_ERR_WORKSPACE;
     if (reinterpret_cast<uintptr_t>(state) % 256 != 0 || reinterpret_cast<uintptr_t>(qkvz) % 4 != 0 ||
         reinterpret_cast<uintptr_t>(ba) % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 4 != 0)
         return SWQ_ERR_MISALIGNED;
+    return SWQ_OK;
+}
+
+extern "C" int swq_deltanet_step(const swq_deltanet_layer *l, const float *qkvz, const float *ba, void *state,
+                                 size_t state_bytes, int64_t position, float *out, void *stream) {
+    const int st = check_step(l, qkvz, ba, state, state_bytes, position, out);
+    if (st != SWQ_OK) return st;
     DnArgs a{};
     a.qkvz = qkvz;
     a.ba = ba;
@@ -331,6 +338,11 @@ extern "C" int swq_deltanet_token(const swq_deltanet_layer *l, const swq_qlinear
     for (int i = 0; i < n_projections; ++i)
         if (projections[i].out_dim > (split ? rows_split : rows_fused)[i]) return SWQ_ERR_BAD_SHAPE;
     if (out_proj->in_dim > val) return SWQ_ERR_BAD_SHAPE;
+    // every check before the first launch: an error leaves the state as it was
+    st = check_gemv_multi(projections, n_projections, ys, x, norm_weight, norm_dtype, norm_eps);
+    if (st == SWQ_OK) st = check_step(l, qkvz, ba, state, state_bytes, position, y);
+    if (st == SWQ_OK) st = check_gemv(out_proj, y, out);
+    if (st != SWQ_OK) return st;
     st = swq_encode_gemv_multi(projections, n_projections, ys, x, norm_weight, norm_dtype, norm_eps, stream);
     if (st == SWQ_OK) st = swq_deltanet_step(l, qkvz, ba, state, state_bytes, position, y, stream);
     if (st == SWQ_OK) st = swq_encode_gemv(out_proj, 0, 0, 0, 0, y, 0, out, 0, stream);

@@ -376,12 +376,9 @@ static int launch_gemv(const swq_qlinear *l, int rows, int64_t w_extra, int64_t 
     return launch_status();
 }
 
-}  // namespace swq
-
-using namespace swq;
-
-extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *const *ys, const float *x,
-                                     const void *norm_weight, int norm_dtype, float norm_eps, void *stream) {
+// The checks of swq_encode_gemv_multi, and its kernel's arguments.
+static int multi_args(const swq_qlinear *lins, int n, float *const *ys, const float *x, const void *norm_weight,
+                      int norm_dtype, float norm_eps, MultiArgs &a, int &total) {
     if (!lins || !ys || !x || n <= 0) return SWQ_ERR_INVALID_ARGUMENT;
     if (n > kMultiMax) return SWQ_ERR_LIMIT;
     if (norm_weight && norm_dtype != SWQ_F32 && norm_dtype != SWQ_F16 && norm_dtype != SWQ_BF16)
@@ -390,7 +387,6 @@ extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *cons
     if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0)
         return SWQ_ERR_MISALIGNED;
     const swq_qlinear &l0 = lins[0];
-    MultiArgs a{};
     for (int i = 0; i < n; ++i) {
         const swq_qlinear &l = lins[i];
         int st = check_linear_shape(&l);
@@ -412,7 +408,7 @@ extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *cons
     if (!(plan_fits(a.m) || q4_wide) || a.m.xf != 0 || a.m.in > kStageMaxIn || a.m.in % 4 != 0)
         return SWQ_ERR_LIMIT;
     const int tile_rows = (4 / a.m.cpl) * (kWave >> a.m.lpr_log2);
-    int total = 0;
+    total = 0;
     for (int i = 0; i < n; ++i) {
         total += (a.rows[i] + tile_rows - 1) / tile_rows;
         a.tile_end[i] = total;
@@ -422,6 +418,32 @@ extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *cons
     a.norm_w = norm_weight;
     a.norm_dtype = norm_dtype;
     a.eps = norm_eps;
+    return SWQ_OK;
+}
+
+int check_gemv_multi(const swq_qlinear *lins, int n, float *const *ys, const float *x, const void *norm_weight,
+                     int norm_dtype, float norm_eps) {
+    MultiArgs a{};
+    int total;
+    return multi_args(lins, n, ys, x, norm_weight, norm_dtype, norm_eps, a, total);
+}
+
+int check_gemv(const swq_qlinear *lin, const float *x, const float *y) {
+    const int st = check_linear_shape(lin);
+    if (st != SWQ_OK) return st;
+    return x && y ? SWQ_OK : SWQ_ERR_INVALID_ARGUMENT;
+}
+
+}  // namespace swq
+
+using namespace swq;
+
+extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *const *ys, const float *x,
+                                     const void *norm_weight, int norm_dtype, float norm_eps, void *stream) {
+    MultiArgs a{};
+    int total;
+    const int st = multi_args(lins, n, ys, x, norm_weight, norm_dtype, norm_eps, a, total);
+    if (st != SWQ_OK) return st;
     const dim3 grid(std::min((total + kGemvThreads / kWave - 1) / (kGemvThreads / kWave), kGemvMaxBlocks));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool f32s = a.m.stype == SWQ_F32, norm = norm_weight != nullptr;
@@ -444,9 +466,9 @@ extern "C" int swq_encode_gemv_multi(const swq_qlinear *lins, int n, float *cons
 extern "C" int swq_encode_gemv(const swq_qlinear *lin, int rows, int64_t w_extra, int64_t s_extra,
                                int64_t b_extra, const float *x, int64_t x_off, float *y, int64_t y_off,
                                void *stream) {
-    int st = check_linear_shape(lin);
+    const int st = check_gemv(lin, x, y);
     if (st != SWQ_OK) return st;
-    if (!x || !y || x_off < 0 || y_off < 0 || w_extra < 0 || s_extra < 0 || b_extra < 0) return SWQ_ERR_INVALID_ARGUMENT;
+    if (x_off < 0 || y_off < 0 || w_extra < 0 || s_extra < 0 || b_extra < 0) return SWQ_ERR_INVALID_ARGUMENT;
     const int n = rows > 0 ? rows : lin->out_dim;
     return launch_gemv(lin, n, w_extra, s_extra, b_extra, x + x_off, y + y_off, true,
                        static_cast<hipStream_t>(stream));

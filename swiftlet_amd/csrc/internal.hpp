@@ -113,4 +113,10 @@ inline QMat make_qmat(const swq_qlinear *l, int64_t w_extra = 0, int64_t s_extra
     return m;
 }
 
+// The checks of swq_encode_gemv_multi and of swq_encode_gemv without offsets (gemv.hip), for
+// calls that have to know before their first launch that the last one will be accepted.
+int check_gemv_multi(const swq_qlinear *lins, int n, float *const *ys, const float *x, const void *norm_weight,
+                     int norm_dtype, float norm_eps);
+int check_gemv(const swq_qlinear *lin, const float *x, const float *y);
+
 }  // namespace swq

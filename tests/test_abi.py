@@ -315,3 +315,53 @@ def test_moe_decode_norm_validation(lib):
     assert call(res=FAKE + (2 << 20), out=FAKE + (2 << 20) + 8) == _lib.SWQ_ERR_INVALID_ARGUMENT  # out overlaps r
     assert call(wsb=ws_bytes - 1) == _lib.SWQ_ERR_WORKSPACE
     assert call(h=FAKE + 2) == _lib.SWQ_ERR_MISALIGNED
+
+
+DELTA = dict(num_key_heads=16, num_value_heads=32, key_head_dim=128, value_head_dim=128, conv_kernel=4,
+             layout=_lib.SWQ_DELTA_SPLIT, norm_eps=1e-6, reserved=0, conv_weight=FAKE, a_log=FAKE, dt_bias=FAKE,
+             norm_weight=FAKE)
+DELTA_ROWS = {_lib.SWQ_DELTA_SPLIT: (8192, 4096, 32, 32), _lib.SWQ_DELTA_INTERLEAVED: (12288, 64)}
+
+
+def delta_token(lib, layout=_lib.SWQ_DELTA_SPLIT, rows=None, out_proj=None, scratch=FAKE, scratch_less=0, state_less=0,
+                x=FAKE, position=0):
+    L = _lib.DeltaNetLayer(**dict(DELTA, layout=layout))
+    rows = rows or DELTA_ROWS[layout]
+    projs = (QLinear * len(rows))(*[lin(n, 2048) for n in rows])
+    n = lib.swq_deltanet_scratch_floats(ctypes.byref(L))
+    return lib.swq_deltanet_token(ctypes.byref(L), projs, len(rows), ctypes.byref(out_proj or lin(2048, 4096)), x, None,
+                                  _lib.SWQ_F32, 1e-6, FAKE, lib.swq_deltanet_state_bytes(ctypes.byref(L)) - state_less,
+                                  position, scratch, n - scratch_less, FAKE, None)
+
+
+def attention_token(lib, rows=(8192, 512, 512), o_proj=None, scratch=FAKE, scratch_less=0, cache_less=0, x=FAKE,
+                    position=0):
+    L = _lib.AttentionLayer(num_heads=16, num_kv_heads=2, head_dim=256, rotary_dims=64, rope_theta=1e7, norm_eps=1e-6,
+                            max_positions=100, reserved=0, q_norm_weight=FAKE, k_norm_weight=FAKE)
+    projs = (QLinear * 3)(*[lin(n, 2048) for n in rows])
+    n = lib.swq_attention_scratch_floats(ctypes.byref(L), projs)
+    return lib.swq_attention_token(ctypes.byref(L), projs, ctypes.byref(o_proj or lin(2048, 4096)), x, None, _lib.SWQ_F32,
+                                   1e-6, FAKE, lib.swq_attention_cache_bytes(ctypes.byref(L)) - cache_less, position,
+                                   scratch, n - scratch_less, FAKE, FAKE,
+                                   lib.swq_attention_workspace_bytes(ctypes.byref(L)), None)
+
+
+def test_token_calls_refuse_before_the_first_launch(lib):
+    """swq_deltanet_token and swq_attention_token check their last launch's arguments too before
+    the first: a refused call has not advanced the recurrence or written a cache row.  (Without a
+    device a launch returns an error of its own, so the code tells which came first.)"""
+    bad_bits, bad_group = lin(2048, 4096, 5), lin(2048, 4096, 4, group=96)
+    null = lin(2048, 4096)
+    null.scales = None
+    for call, key in ((delta_token, "out_proj"), (attention_token, "o_proj")):
+        assert call(lib, **{key: bad_bits}) == _lib.SWQ_ERR_UNSUPPORTED_BITS
+        assert call(lib, **{key: bad_group}) == _lib.SWQ_ERR_BAD_SHAPE
+        assert call(lib, **{key: null}) == _lib.SWQ_ERR_INVALID_ARGUMENT
+        assert call(lib, **{key: lin(2048, 8192)}) == _lib.SWQ_ERR_BAD_SHAPE  # reads past the step's output
+        assert call(lib, x=FAKE + 4) == _lib.SWQ_ERR_MISALIGNED
+        assert call(lib, position=-1) == _lib.SWQ_ERR_INVALID_ARGUMENT
+        assert call(lib, scratch_less=1) == _lib.SWQ_ERR_WORKSPACE
+    assert delta_token(lib, state_less=1) == _lib.SWQ_ERR_WORKSPACE
+    assert attention_token(lib, cache_less=1) == _lib.SWQ_ERR_WORKSPACE
+    assert attention_token(lib, position=100) == _lib.SWQ_ERR_LIMIT
+    assert attention_token(lib, rows=(8192, 512, 511)) == _lib.SWQ_ERR_BAD_SHAPE
