@@ -593,6 +593,7 @@ extern "C" int swq_attention_token(const swq_attention_layer *l, const swq_qline
         o_proj->in_dim > val)
         return SWQ_ERR_BAD_SHAPE;
     if (scratch_floats < swq_attention_scratch_floats(l, projections)) return SWQ_ERR_WORKSPACE;
+    if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return SWQ_ERR_MISALIGNED;
     float *q = scratch, *k = q + pad_floats(projections[0].out_dim), *v = k + pad_floats(projections[1].out_dim);
     float *y = v + pad_floats(projections[2].out_dim);
     float *ys[3] = {q, k, v};

@@ -330,6 +330,7 @@ extern "C" int swq_deltanet_token(const swq_deltanet_layer *l, const swq_qlinear
     const int64_t nv = l->num_value_heads, val = nv * l->value_head_dim;
     const int64_t conv = 2LL * l->num_key_heads * l->key_head_dim + val;
     if (scratch_floats < swq_deltanet_scratch_floats(l)) return SWQ_ERR_WORKSPACE;
+    if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return SWQ_ERR_MISALIGNED;
     float *qkvz = scratch, *ba = qkvz + pad_floats(conv + val), *y = ba + pad_floats(2 * nv);
     const bool split = l->layout == SWQ_DELTA_SPLIT;
     float *ys[4] = {qkvz, split ? qkvz + conv : ba, ba, ba + nv};

@@ -365,3 +365,10 @@ def test_token_calls_refuse_before_the_first_launch(lib):
     assert attention_token(lib, cache_less=1) == _lib.SWQ_ERR_WORKSPACE
     assert attention_token(lib, position=100) == _lib.SWQ_ERR_LIMIT
     assert attention_token(lib, rows=(8192, 512, 511)) == _lib.SWQ_ERR_BAD_SHAPE
+
+
+def test_token_scratch_alignment(lib):
+    for call in (delta_token, attention_token):
+        for off in (1, 4, 8):
+            assert call(lib, scratch=FAKE + off) == _lib.SWQ_ERR_MISALIGNED
+        assert call(lib, scratch=None) == _lib.SWQ_ERR_INVALID_ARGUMENT
