@@ -266,9 +266,11 @@ int swq_deltanet_step(const swq_deltanet_layer *layer, const float *qkvz, const 
 
 /* The whole block for one token in one call: the projections of x (one launch;
  * with norm_weight, x is the un-normalised hidden state), swq_deltanet_step and
- * out_proj (f32 out).  projections: SPLIT qkv, z, b, a; INTERLEAVED qkvz, ba.
+ * out_proj (at most nv*dv inputs; f32 out).  projections: SPLIT qkv, z, b, a;
+ * INTERLEAVED qkvz, ba, each with exactly the rows that the step reads.
  * scratch: swq_deltanet_scratch_floats(layer) f32 device words, 16-byte
- * aligned, dead after the call's work. */
+ * aligned, dead after the call's work.  An error is returned before the first
+ * launch: the state is then unchanged. */
 size_t swq_deltanet_scratch_floats(const swq_deltanet_layer *layer);
 int swq_deltanet_token(const swq_deltanet_layer *layer, const swq_qlinear *projections, int n_projections,
                        const swq_qlinear *out_proj, const float *x, const void *norm_weight, int norm_dtype,
@@ -316,9 +318,10 @@ int swq_attention_step(const swq_attention_layer *layer, const float *q_proj, co
 
 /* The whole block for one token in one call: q/k/v_proj of x (one launch; with
  * norm_weight, x is the un-normalised hidden state), swq_attention_step and
- * o_proj (f32 out).  projections: q, k, v, of at least 2*H*hd, KVH*hd and
- * KVH*hd rows.  scratch: swq_attention_scratch_floats f32 device words, 16-byte
- * aligned, dead after the call's work. */
+ * o_proj (at most H*hd inputs; f32 out).  projections: q, k, v, of at least
+ * 2*H*hd, KVH*hd and KVH*hd rows.  scratch: swq_attention_scratch_floats f32
+ * device words, 16-byte aligned, dead after the call's work.  An error is
+ * returned before the first launch: the cache is then unchanged. */
 size_t swq_attention_scratch_floats(const swq_attention_layer *layer, const swq_qlinear *projections);
 int swq_attention_token(const swq_attention_layer *layer, const swq_qlinear *projections,
                         const swq_qlinear *o_proj, const float *x, const void *norm_weight, int norm_dtype,

@@ -337,7 +337,7 @@ extern "C" int swq_deltanet_token(const swq_deltanet_layer *l, const swq_qlinear
     const int64_t rows_split[4] = {conv, val, nv, nv}, rows_fused[2] = {conv + val, 2 * nv};
     if (n_projections != (split ? 4 : 2)) return SWQ_ERR_BAD_SHAPE;
     for (int i = 0; i < n_projections; ++i)
-        if (projections[i].out_dim > (split ? rows_split : rows_fused)[i]) return SWQ_ERR_BAD_SHAPE;
+        if (projections[i].out_dim != (split ? rows_split : rows_fused)[i]) return SWQ_ERR_BAD_SHAPE;
     if (out_proj->in_dim > val) return SWQ_ERR_BAD_SHAPE;
     // every check before the first launch: an error leaves the state as it was
     st = check_gemv_multi(projections, n_projections, ys, x, norm_weight, norm_dtype, norm_eps);

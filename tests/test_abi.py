@@ -372,3 +372,15 @@ def test_token_scratch_alignment(lib):
         for off in (1, 4, 8):
             assert call(lib, scratch=FAKE + off) == _lib.SWQ_ERR_MISALIGNED
         assert call(lib, scratch=None) == _lib.SWQ_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("layout", [_lib.SWQ_DELTA_SPLIT, _lib.SWQ_DELTA_INTERLEAVED], ids=["split", "interleaved"])
+def test_deltanet_token_needs_every_row(lib, layout):
+    """A projection with too few rows would leave scratch words that the step reads unwritten, one
+    with too many would write into the next one's."""
+    rows = DELTA_ROWS[layout]
+    for i in range(len(rows)):
+        for d in (-1, 1):
+            bad = rows[:i] + (rows[i] + d,) + rows[i + 1:]
+            assert delta_token(lib, layout=layout, rows=bad) == _lib.SWQ_ERR_BAD_SHAPE, bad
+    assert delta_token(lib, layout=layout, rows=rows[:-1]) == _lib.SWQ_ERR_BAD_SHAPE
