@@ -11,7 +11,8 @@ import ctypes
 
 from . import _lib
 from ._lib import AttentionLayer, check
-from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch
+from .engine import (ENGINE_LAUNCHES, DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch,
+                     replaced)
 
 
 class AttentionGPU:
@@ -76,10 +77,14 @@ class AttentionGPU:
                       stream=None):
         """x [H_model] f32 -> the block's output: q/k/v_proj in one launch
         (with norm_weight, x is the un-normalised hidden state and the input
-        RMSNorm runs inside that launch), the step, o_proj."""
+        RMSNorm runs inside that launch), the step, o_proj.  One native call,
+        or the launches one by one where `step` or one of the engine's has been
+        overridden."""
         if _elsewhere(stream):
             with _torch().cuda.stream(stream):
-                return self.forward_token(engine, x, cache, ws, position, norm_weight, eps)
+                return AttentionGPU.forward_token(self, engine, x, cache, ws, position, norm_weight, eps)
+        if replaced(engine, ENGINE_LAUNCHES) or replaced(self, _STEP):
+            return self._forward_launches(engine, x, cache, ws, position, norm_weight, eps, stream)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         pq, pk, pv = self.projections
         projs = self._projs.of((pq, pk, pv))
@@ -92,6 +97,18 @@ class AttentionGPU:
             cache.numel(), position, scratch.data_ptr(), n, r.data_ptr(), ws.data_ptr(), ws.numel(),
             _stream_handle(stream)), "attention_token")
         return r
+
+    def _forward_launches(self, engine, x, cache, ws, position, norm_weight, eps, stream):
+        torch = _torch()
+        q, k, v = (torch.empty(p.out_dim, dtype=torch.float32, device=x.device) for p in self.projections)
+        engine.encode_gemv_multi(list(self.projections), x, [q, k, v], norm_weight=norm_weight, eps=eps, stream=stream)
+        att = self.step(q, k, v, cache, ws, position, stream=stream)
+        r = torch.empty(self.o_proj.out_dim, dtype=torch.float32, device=x.device)
+        engine.encode_gemv(self.o_proj, att, r, stream=stream)
+        return r
+
+
+_STEP = (("step", AttentionGPU.step),)
 
 
 def attention_from_checkpoint(ckpt, layer: int, config: dict, max_positions: int = 4096, device="cuda",

@@ -10,7 +10,8 @@ import ctypes
 
 from . import _lib
 from ._lib import SWQ_DELTA_INTERLEAVED, SWQ_DELTA_SPLIT, DeltaNetLayer, check
-from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch
+from .engine import (ENGINE_LAUNCHES, DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch,
+                     replaced)
 
 
 class DeltaNetGPU:
@@ -81,10 +82,14 @@ class DeltaNetGPU:
                       stream=None):
         """x [H] f32 -> the block's output [H]: the input projections in one
         launch (with norm_weight, x is the un-normalised hidden state and the
-        input RMSNorm runs inside that launch), the step, out_proj."""
+        input RMSNorm runs inside that launch), the step, out_proj.  One native
+        call, or the launches one by one where `step` or one of the engine's
+        has been overridden."""
         if _elsewhere(stream):
             with _torch().cuda.stream(stream):
-                return self.forward_token(engine, x, state, position, norm_weight, eps)
+                return DeltaNetGPU.forward_token(self, engine, x, state, position, norm_weight, eps)
+        if replaced(engine, ENGINE_LAUNCHES) or replaced(self, _STEP):
+            return self._forward_launches(engine, x, state, position, norm_weight, eps, stream)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         scratch = empty(self._scratch, dtype=f32, device=dev)
         r = empty(self.out_proj.out_dim, dtype=f32, device=dev)
@@ -94,6 +99,23 @@ class DeltaNetGPU:
             x.data_ptr(), wptr, wdt, eps, state.data_ptr(), state.numel(), position, scratch.data_ptr(), self._scratch,
             r.data_ptr(), _stream_handle(stream)), "deltanet_token")
         return r
+
+    def _forward_launches(self, engine, x, state, position, norm_weight, eps, stream):
+        torch = _torch()
+        qkvz = torch.empty(self.conv_dim + self.value_dim, dtype=torch.float32, device=x.device)
+        ba = torch.empty(2 * self.nv, dtype=torch.float32, device=x.device)
+        if self.layout == SWQ_DELTA_INTERLEAVED:
+            ys = [qkvz, ba]
+        else:
+            ys = [qkvz.data_ptr(), qkvz.data_ptr() + 4 * self.conv_dim, ba.data_ptr(), ba.data_ptr() + 4 * self.nv]
+        engine.encode_gemv_multi(list(self.projections), x, ys, norm_weight=norm_weight, eps=eps, stream=stream)
+        y = self.step(qkvz, ba, state, position, stream=stream)
+        r = torch.empty(self.out_proj.out_dim, dtype=torch.float32, device=x.device)
+        engine.encode_gemv(self.out_proj, y, r, stream=stream)
+        return r
+
+
+_STEP = (("step", DeltaNetGPU.step),)
 
 
 def deltanet_from_checkpoint(ckpt, layer: int, config: dict, device="cuda", stream=None) -> DeltaNetGPU:

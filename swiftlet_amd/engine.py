@@ -242,7 +242,8 @@ class HipEngine:
         vocab = logits.numel()
         if _elsewhere(stream):
             with torch.cuda.stream(stream):
-                return self.sample(logits, temperature, top_k, top_p, presence, frequency, seen, banned, u, ws)
+                return HipEngine.sample(self, logits, temperature, top_k, top_p, presence, frequency, seen, banned, u,
+                                        ws)
         if ws is None:
             ws = self.new_sample_workspace(vocab, dev)
         seen, banned = seen or {}, list(banned)
@@ -273,3 +274,16 @@ class HipEngine:
         check(self.lib.swq_dequantize(ctypes.byref(c), row0, rows, out.data_ptr(),
                                       _stream_handle(stream)), "dequantize")
         return out
+
+
+# the launches that a block's forward_token makes in one native call instead
+ENGINE_LAUNCHES = (("encode_gemv", HipEngine.encode_gemv), ("encode_gemv_multi", HipEngine.encode_gemv_multi))
+
+
+def replaced(obj, methods) -> bool:
+    """Whether `obj` has another function than its class's own under one of these names: a
+    subclass's, an instance's, or one put in place of the class's."""
+    for name, own in methods:
+        if getattr(getattr(obj, name, None), "__func__", None) is not own:
+            return True
+    return False

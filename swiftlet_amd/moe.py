@@ -162,7 +162,7 @@ class MoELayerGPU:
         torch = _torch()
         if _elsewhere(stream):
             with torch.cuda.stream(stream):
-                return self.new_prefill_workspace(tokens)
+                return MoELayerGPU.new_prefill_workspace(self, tokens)
         n = self.prefill_workspace_bytes(tokens)
         ws = torch.empty(n, dtype=torch.uint8, device=self.router.w.device)
         check(self.lib.swq_moe_workspace_init(ws.data_ptr(), n, _stream_handle(stream)), "workspace_init")

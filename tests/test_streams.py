@@ -4,98 +4,45 @@ Without a device, on stand-ins for torch and the library that record which strea
 each allocation; on a device, against the call on the current stream while that stream allocates
 and overwrites blocks of the same size."""
 
-import contextlib
-import types
-
 import pytest
 
 from swiftlet_amd import attention, deltanet, engine, moe
+from tests import fakes
 
 
-class FakeTorch:
-    """empty() and the current stream of torch; `log` holds the stream of each allocation."""
-
-    float32, bfloat16, int32, uint8 = "f32", "bf16", "i32", "u8"
-
-    def __init__(self):
-        self.current, self.log = types.SimpleNamespace(cuda_stream="default"), []
-        self.cuda = types.SimpleNamespace(current_stream=lambda: self.current, stream=self._stream,
-                                          current_device=lambda: 0)
-        self._C = types.SimpleNamespace(_cuda_getCurrentRawStream=lambda device: self.current.cuda_stream)
-
-    @contextlib.contextmanager
-    def _stream(self, s):
-        before, self.current = self.current, s
-        yield
-        self.current = before
-
-    def empty(self, n, dtype=None, device=None):
-        self.log.append(self.current.cuda_stream)
-        return types.SimpleNamespace(data_ptr=lambda: 0x1000, dtype=dtype, numel=lambda: n)
+@pytest.fixture
+def fake(monkeypatch):
+    f = fakes.FakeTorch()
+    for m in (engine, deltanet, attention, moe):
+        monkeypatch.setattr(m, "_torch", lambda: f)
+    return f
 
 
-class FakeLib:
-    """Every entry returns success; `streams` holds the last argument of the token and prefill calls."""
-
-    def __init__(self):
-        self.streams = []
-
-    def __getattr__(self, name):
-        def call(*args):
-            if name.endswith(("_token", "_prefill")):
-                self.streams.append(args[-1])
-            return 64 if name.endswith(("_floats", "_bytes")) else 0
-        return call
-
-
-def _lin():
-    t = types.SimpleNamespace(data_ptr=lambda: 0x2000)
-    return engine.GPULinear(t, t, t, 64, 64, 64, 4, 0)
-
-
-def _block(cls, **fields):
-    blk = cls.__new__(cls)
-    blk._c = (deltanet.DeltaNetLayer if cls is deltanet.DeltaNetGPU else attention.AttentionLayer)()
-    blk.lib, blk._projs, blk._scratch = FakeLib(), engine.DescArray(), 64
-    for k, v in fields.items():
-        setattr(blk, k, v)
-    return blk
-
-
-@pytest.mark.parametrize("kind", ["delta", "attention"])
-def test_token_scratch_is_allocated_on_the_given_stream(kind, monkeypatch):
-    fake = FakeTorch()
-    for m in (engine, deltanet, attention):
-        monkeypatch.setattr(m, "_torch", lambda: fake)
-    eng = engine.HipEngine.__new__(engine.HipEngine)
-    buf = types.SimpleNamespace(data_ptr=lambda: 0x3000, device="cuda", numel=lambda: 64, dtype="f32")
-    if kind == "delta":
-        blk = _block(deltanet.DeltaNetGPU, projections=(_lin(),) * 4, out_proj=_lin())
-        call = lambda s: blk.forward_token(eng, buf, buf, 0, stream=s)  # noqa: E731
-    else:
-        blk = _block(attention.AttentionGPU, projections=(_lin(),) * 3, o_proj=_lin())
-        call = lambda s: blk.forward_token(eng, buf, buf, buf, 0, stream=s)  # noqa: E731
-    call(None)
-    assert fake.log == ["default"] * 2 and blk.lib.streams == ["default"]
-    call(types.SimpleNamespace(cuda_stream="side"))
-    assert fake.log == ["default"] * 2 + ["side"] * 2 and blk.lib.streams == ["default", "side"]
+@pytest.mark.parametrize("cls,entry", [(deltanet.DeltaNetGPU, "swq_deltanet_token"),
+                                       (attention.AttentionGPU, "swq_attention_token")])
+def test_token_scratch_is_allocated_on_the_given_stream(fake, cls, entry):
+    lib = fakes.FakeLib()
+    _, token = fakes.block(cls, lib)
+    eng = fakes.hip_engine(lib)
+    token(eng)
+    assert fake.log == ["default"] * 2 and lib.calls == [(entry, "default")]
+    token(eng, fakes.SIDE)
+    assert fake.log == ["default"] * 2 + ["side"] * 2 and lib.calls[1:] == [(entry, "side")]
     assert fake.current.cuda_stream == "default"
 
 
-def test_prefill_workspace_is_allocated_on_the_given_stream(monkeypatch):
+def test_prefill_workspace_is_allocated_on_the_given_stream(fake):
     """A prefill without a workspace makes one and lets go of it on return."""
-    fake = FakeTorch()
-    for m in (engine, moe):
-        monkeypatch.setattr(m, "_torch", lambda: fake)
     layer = moe.MoELayerGPU.__new__(moe.MoELayerGPU)
-    layer._c, layer.lib, layer.router, layer.hidden, layer.top_k = moe.MoELayer(), FakeLib(), _lin(), 64, 2
-    layer.router.w.device = "cuda"
-    buf = types.SimpleNamespace(data_ptr=lambda: 0x3000, device="cuda", dtype="f32", shape=(1, 64), dim=lambda: 2)
+    lib = fakes.FakeLib()
+    layer._c, layer.lib, layer.router, layer.hidden, layer.top_k = moe.MoELayer(), lib, fakes.linear(), 64, 2
+    buf = fakes.tensor()
+    buf.shape, buf.dim = (1, 64), lambda: 2
     given = dict(out=buf, topk_ids=buf, topk_weights=buf)
     layer.prefill(buf, **given)
-    assert fake.log == ["default"] and layer.lib.streams == ["default"]
-    layer.prefill(buf, stream=types.SimpleNamespace(cuda_stream="side"), **given)
-    assert fake.log == ["default", "side"] and layer.lib.streams == ["default", "side"]
+    layer.prefill(buf, stream=fakes.SIDE, **given)
+    assert fake.log == ["default", "side"]
+    assert lib.calls == [(n, s) for s in ("default", "side") for n in ("swq_moe_workspace_init", "swq_moe_prefill")]
 
 
 @pytest.mark.gpu
