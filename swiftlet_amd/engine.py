@@ -28,11 +28,13 @@ def _torch():
 
 def _stream_handle(stream) -> int:
     """The raw stream of a torch stream, or of the current one; without building a torch stream
-    object for the latter, which costs a launch's host time again."""
+    object for the latter, which costs a launch's host time again, where torch has the (private)
+    entry for it."""
     if stream is not None:
         return stream.cuda_stream
-    cuda = _torch().cuda
-    return _torch()._C._cuda_getCurrentRawStream(cuda.current_device())
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(torch.cuda.current_device()) if raw else torch.cuda.current_stream().cuda_stream
 
 
 def _elsewhere(stream) -> bool:

@@ -45,6 +45,13 @@ def test_prefill_workspace_is_allocated_on_the_given_stream(fake):
     assert lib.calls == [(n, s) for s in ("default", "side") for n in ("swq_moe_workspace_init", "swq_moe_prefill")]
 
 
+def test_current_stream_without_torchs_private_entry(fake):
+    """The raw current stream where this torch lacks the entry that returns it directly."""
+    assert engine._stream_handle(None) == "default"
+    del fake._C._cuda_getCurrentRawStream
+    assert engine._stream_handle(None) == "default" and engine._stream_handle(fakes.SIDE) == "side"
+
+
 @pytest.mark.gpu
 def test_token_on_a_side_stream_while_the_current_one_reuses_memory():
     """Both blocks on a side stream that is still busy when the call returns, while the current
