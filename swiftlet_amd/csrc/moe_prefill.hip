@@ -1714,8 +1714,13 @@ int router_kslices(int H) { return (H / kGroupK + kBlockG - 1) / kBlockG; }
 //   512 experts top-10, 4-bit 113/98 161/139 196/171 221/200 237/223 309/316
 // (f32 x at 256 tokens, 4-bit: 165/170.)
 constexpr int kThinAvgRows = 6;
-bool thin_tiles(const swq_moe_layer *l, int T) {
-    return T <= kThinRows || static_cast<int64_t>(T) * l->top_k <= static_cast<int64_t>(kThinAvgRows) * l->num_experts;
+int most_thin_tokens(const swq_moe_layer *l) { return std::max(kThinRows, kThinAvgRows * l->num_experts / l->top_k); }
+bool thin_tiles(const swq_moe_layer *l, int T) { return T <= most_thin_tokens(l); }
+
+// Most tiles of up to `cap` rows that T tokens can make.
+int most_tiles(const swq_moe_layer *l, int T, int cap) {
+    const size_t P = static_cast<size_t>(T) * l->top_k, U = std::min<size_t>(P, static_cast<size_t>(l->num_experts));
+    return static_cast<int>((P + static_cast<size_t>(cap - 1) * U) / cap) + (l->has_shared ? (T + cap - 1) / cap : 0);
 }
 
 // From kRouterWide tokens on the router's tiles have twice the rows, which halves the passes
@@ -1741,10 +1746,10 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
     };
     const size_t P = static_cast<size_t>(T) * l->top_k;
     const size_t rows = P + (l->has_shared ? T : 0);
-    const int U = static_cast<int>(std::min<size_t>(P, static_cast<size_t>(l->num_experts)));
-    const int cap = thin_tiles(l, T) ? kThinRows : kTileRows;
-    w.max_tiles = static_cast<int>((P + static_cast<size_t>(cap - 1) * U) / cap) +
-                  (l->has_shared ? (T + cap - 1) / cap : 0);
+    // the table has room for what any T' <= T needs, in either tile size, so that a workspace
+    // made for T tokens serves fewer too
+    const int thin = most_tiles(l, std::min(T, most_thin_tokens(l)), kThinRows);
+    w.max_tiles = thin_tiles(l, T) ? thin : most_tiles(l, T, kTileRows);
     w.Ih = std::max(l->moe_intermediate, l->has_shared ? l->shared_intermediate : 0);
     w.header = take(256);  // [1] tile count
     w.counts = P > kGroupSplitPairs ? take(static_cast<size_t>(kGroupSplit) * l->num_experts * 4) : 0;
@@ -1755,7 +1760,7 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
     w.wts = take(P * 4);
     w.pos = take(P * 4);
     w.tok = take(rows * 4);
-    w.tiles = take(static_cast<size_t>(w.max_tiles) * sizeof(Tile));
+    w.tiles = take(static_cast<size_t>(std::max(thin, w.max_tiles)) * sizeof(Tile));
     w.xs_ld_x = ((l->hidden / kGroupK) + 31) & ~31;  // whole 32-group blocks (the bias MFMA's k)
     w.xs_ld_h = ((w.Ih / kGroupK) + 31) & ~31;
     w.xs_x = take(static_cast<size_t>(T) * w.xs_ld_x * 4);

@@ -207,6 +207,16 @@ def test_prefill_workspace_query(lib):
     assert lib.swq_moe_prefill_workspace_bytes(ctypes.byref(layer(router=lin(256, 2048, 8, group=32))), 8) == 0
 
 
+@pytest.mark.parametrize("E,K,H,I", [(1023, 1, 128, 128), (721, 1, 128, 128), (1024, 4, 128, 128), (8, 2, 128, 128),
+                                     (1, 1, 128, 128), (256, 8, 2048, 512), (512, 10, 2048, 512)])
+def test_prefill_workspace_serves_fewer_tokens(lib, E, K, H, I):
+    """The bytes never fall as the tokens grow, also where the tiles change from 16 rows to 64 (6 E / K
+    tokens) and where the grouping changes: a workspace made for a chunk takes every smaller one."""
+    L = layer(H=H, E=E, K=K, I=I, Is=I)
+    n = [lib.swq_moe_prefill_workspace_bytes(ctypes.byref(L), t) for t in range(1, 9000)]
+    assert n[0] > 0 and all(a <= b for a, b in zip(n, n[1:]))
+
+
 @pytest.mark.parametrize("mutate,code", [
     (dict(router=lin(256, 2048, 8, group=32)), _lib.SWQ_ERR_LIMIT),        # group 64 only
     (dict(I=64, Is=64), _lib.SWQ_ERR_LIMIT),                                # down rows of 64 inputs
