@@ -795,30 +795,18 @@ __device__ __forceinline__ void ring_wait() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
-// ring_wait<Cn>() for the wave's count n of live activation copies per
-// group (wave-uniform, 0..4): one branch per count, each with its immediate.
-template <int C0, int C1, int C2, int C3, int C4>
-__device__ __forceinline__ void ring_wait_sel(int n) {
-    if (n <= 0) ring_wait<C0>();
-    else if (n == 1) ring_wait<C1>();
-    else if (n == 2) ring_wait<C2>();
-    else if (n == 3) ring_wait<C3>();
-    else ring_wait<C4>();
-}
-
 // The grouped quantised GEMM of pf_gemm (same tile, lanes and arithmetic) fed
-// by an LDS ring D groups deep: per group, each wave's DMA brings in its
-// share of the 64 activation rows (NPL bf16 planes, already in the order the
-// codes need) and its 2 x 16 code rows (f32 scales: and their scales); a
-// group is used D - 1 groups after its loads were issued.  2-byte scales come
+// by LDS rings: per group, each wave's DMA brings in its share of the 64
+// activation rows (NPL bf16 planes, already in the order the codes need) one
+// group ahead of its use and its 2 x 16 code rows (f32 scales: and their
+// scales) two groups ahead.  2-byte scales come
 // from registers: the bias term's scale preload holds every group's, handed
 // between lanes per group.  Activation rows are 128 B; row r
 // keeps its 16 B chunk c in slot c ^ (r & 7) so the matrix-core reads of 16
 // rows at one chunk hit distinct banks.
-template <int BITS, int ST, int NPL, int EPI, int DA, int DB, int WAVES>
+template <int BITS, int ST, int NPL, int EPI, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void pf_gemm_dma(const GemmArgs a) {
-    // B(g) must be issued before A(g) for the wait on A(g) to cover it
-    static_assert(DA >= 2 && DB > DA, "ring depths");
+    constexpr int DA = 2, DB = 3;                    // groups in the rings of activations and codes
     static_assert(WAVES == 4 || WAVES == 8, "waves per workgroup");
     constexpr int MT = 4, ROWS = 64;
     constexpr int AW = 8 / WAVES;                    // 8-row slabs each wave brings in per plane
@@ -826,8 +814,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     constexpr int B_WAVE = BITS == 4 ? 1024 : 2048;  // code bytes per wave per group
     constexpr bool kScaleDma = ST == SWQ_F32;        // f32 scales ride the ring
     constexpr int B_SLOT = WAVES * (B_WAVE + (kScaleDma ? 256 : 0));  // codes (+ scales) of one group
-    // DMA instructions per wave per group: activations, codes (+ scales)
-    constexpr int LA = AW * NPL, LB = B_WAVE / 1024 + (kScaleDma ? 1 : 0), L = LA + LB;
+    constexpr int LB = B_WAVE / 1024 + (kScaleDma ? 1 : 0);  // DMA instructions of issue_b
     __shared__ __attribute__((aligned(16))) uint8_t s_ring_a[DA * A_SLOT];
     __shared__ __attribute__((aligned(16))) uint8_t s_ring_b[DB * B_SLOT];
     __shared__ __attribute__((aligned(16))) uint8_t s_xs[ROWS * 128];  // group sums of the rows
@@ -881,9 +868,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     const uint8_t *xsrc[AW];
     // rows past the tile are not fetched (their LDS rows hold stale values,
     // which stay in those rows of the matrix-core results, never stored):
-    // a wave issues the copies of its slabs that hold tile rows (`live`, the
-    // same count every group; the ring waits use it), and within a partial
-    // slab lane 0 always fetches so that no copy is empty
+    // a wave issues the copies of its slabs that hold tile rows (`live`), and
+    // within a partial slab lane 0 always fetches so that no copy is empty
     const int live = min(AW, max(0, (rows + 7) / 8 - AW * wave));
     bool afetch[AW];
 #pragma unroll
@@ -922,7 +908,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     BiasBS<ST> bi;
     load_bias_bs<ST>(bi, sbase, bbase, srow, NG, kg);
 
-    // group g's activation rows into A slot sa (LA instructions per wave)
+    // group g's activation rows into A slot sa (NPL * live instructions)
     auto issue_a = [&](int sa, int g) {
         const uint32_t base = ring_a + sa * A_SLOT;
 #pragma unroll
@@ -1013,37 +999,22 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
     }
 
-    // ---- the rings: codes DB-1 groups ahead, activation rows
-    // (mostly L2 hits) DA-1 groups ahead.  Before the loop: B groups 0..DB-2,
-    // then A groups 0..DA-2.  At group g: wait until A(g) has landed (B(g)
-    // is older), then refill the slots group g-1 used with A(g+DA-1) and
-    // B(g+DB-1) (past NG: group NG-1 again, never read), then compute g.
-    // Loads return in order, so "at most N of this wave's loads in flight"
-    // with N = the loads issued after A(g) means A(g) and everything before
-    // it have landed; N is the same for every group from DA-1 on, and the
-    // first DA-1 groups are peeled with their own counts.  The counts depend
-    // on the wave's live copies n = NPL * live per group: with none, the same
-    // formula counts the loads after B(g) (issued one step before A(g)
-    // would be, DB = DA + 1) exactly in the loop and too few in the peeled
-    // groups (a stricter wait).
+    // ---- the rings: activation rows (mostly L2 hits) one group ahead, codes
+    // two.  Before the loop: B groups 0 and 1, then A group 0.  At group g: wait
+    // until A(g) has landed (B(g) is older), then refill the slots group g-1 used
+    // with A(g+1) and B(g+2) (past NG: group NG-1 again, never read), then
+    // compute g.  Loads return in order, and those issued after A(g) are B(g+1)'s
+    // LB, so at most LB in flight means that A(g) and everything before it have
+    // landed (without a live slab too: B(g) is older than B(g+1)).
 #pragma unroll
     for (int s = 0; s < DB - 1; ++s) issue_b(s, min(s, NG - 1));
-#pragma unroll
-    for (int s = 0; s < DA - 1; ++s) issue_a(s, min(s, NG - 1));
+    issue_a(0, 0);
     auto step = [&](int g, int sa, int sb) {
-        issue_a(sa == 0 ? DA - 1 : sa - 1, min(g + DA - 1, NG - 1));
+        issue_a(sa ^ 1, min(g + 1, NG - 1));
         issue_b(sb == 0 ? DB - 1 : sb - 1, min(g + DB - 1, NG - 1));
         compute(sa, sb, g);
     };
-    static_assert(DA <= 4 && DB == DA + 1 && LA <= 4, "peeled prologue, wait counts");
-    const int nl = NPL * live;
-    // the wait counts for n live copies per group (n <= LA)
-    constexpr auto w0 = [](int n) constexpr { return (DA - 2) * n; };
-    constexpr auto w1 = [](int n) constexpr { return (DA - 3) * n + (n + LB); };
-    constexpr auto w2 = [](int n) constexpr { return (DA - 4) * n + 2 * (n + LB); };
-    constexpr auto wl = [](int n) constexpr { return LB + (DA - 2) * (n + LB); };
-    constexpr auto cl = [](int n) constexpr { return n < LA ? n : LA; };
-    if (0 < NG) ring_wait_sel<w0(0), w0(cl(1)), w0(cl(2)), w0(cl(3)), w0(cl(4))>(nl);
+    if (0 < NG) ring_wait<0>();
     // The scale words were loaded before every ring load, so the wait above
     // has landed them; the compiler cannot know that (it does not count the
     // DMA loads) and would wait for them at their first use in the loop, on
@@ -1058,23 +1029,13 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bi.s[j][i]));
     if (0 < NG) step(0, 0, 0);
-    if constexpr (DA >= 3)
-        if (1 < NG) {
-            ring_wait_sel<w1(0), w1(cl(1)), w1(cl(2)), w1(cl(3)), w1(cl(4))>(nl);
-            step(1, 1, 1);
-        }
-    if constexpr (DA >= 4)
-        if (2 < NG) {
-            ring_wait_sel<w2(0), w2(cl(1)), w2(cl(2)), w2(cl(3)), w2(cl(4))>(nl);
-            step(2, 2, 2);
-        }
     {
-        int sa = (DA - 1) % DA, sb = (DA - 1) % DB;
+        int sa = 1, sb = 1;
 #pragma unroll 1
-        for (int g = DA - 1; g < NG; ++g) {
-            ring_wait_sel<wl(0), wl(cl(1)), wl(cl(2)), wl(cl(3)), wl(cl(4))>(nl);
+        for (int g = 1; g < NG; ++g) {
+            ring_wait<LB>();
             step(g, sa, sb);
-            sa = sa + 1 == DA ? 0 : sa + 1;
+            sa ^= 1;
             sb = sb + 1 == DB ? 0 : sb + 1;
         }
     }
@@ -1105,7 +1066,9 @@ constexpr int kThinRows = 16;
 // 32-byte pieces and pays a barrier and an LDS round trip per group.  Here a
 // ring stage is 128 bytes of every code row, whole cache lines (four groups of
 // 4-bit codes, two of 8-bit ones), next to the 16 activation rows of those
-// groups; S stages.  Row r's 16-byte chunk c sits in slot c ^ (r & 7) of its
+// groups; two stages (43 to 68 KB of LDS, two or three workgroups per CU; three
+// stages measured 36 against 34 us for gate/up and 37 against 25 us for down,
+// 16 tokens, 256 experts top-8, 4-bit).  Row r's 16-byte chunk c sits in slot c ^ (r & 7) of its
 // 128 bytes, codes and activations alike.
 //
 // Bound: the codes' bytes, then (one token) the latency of a workgroup's eight
@@ -1115,13 +1078,13 @@ constexpr int kThinRows = 16;
 // waves, 60 and 35 us at 16 tokens; one-wave workgroups, 256-byte row pieces
 // in 32 KB of LDS, 57 and 45; the single-group ring with 16-row activation
 // slots six groups deep, 42 and 26.
-template <int BITS, int ST, int NPL, int EPI, int S>
+template <int BITS, int ST, int NPL, int EPI>
 __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
     constexpr int WAVES = 4, GPS = BITS == 4 ? 4 : 2;  // groups per stage
     constexpr int A_GROUP = NPL * kThinRows * 128, A_STAGE = GPS * A_GROUP;
     constexpr int B_WAVE = 4096, B_STAGE = WAVES * B_WAVE;
-    __shared__ __attribute__((aligned(16))) uint8_t s_ring_a[S * A_STAGE];
-    __shared__ __attribute__((aligned(16))) uint8_t s_ring_b[S * B_STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring_a[2 * A_STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring_b[2 * B_STAGE];
     __shared__ __attribute__((aligned(16))) uint8_t s_xs[kThinRows * 128];
     __shared__ float s_red[EPI == kEpiSwiGLU ? WAVES * kThinRows : 1];
 
@@ -1172,7 +1135,6 @@ __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
     const int slabs = rows > 8 ? 2 : 1;
     const int au = BITS == 4 ? wave : wave >> 1, as0 = BITS == 4 ? 0 : wave & 1;
     const int as1 = BITS == 4 ? slabs : min(as0 + 1, slabs);  // slabs [as0, as1)
-    const int na = max(0, as1 - as0) * NPL;
     const uint8_t *asrc[2], *xsrc[2];
     bool fetch[2];
 #pragma unroll
@@ -1261,18 +1223,13 @@ __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
         }
     };
 
-    // ---- the ring: stages 0 .. S-2 first; at stage st, wait until it has
-    // landed (the newest min(S - 2, NS - 1 - st) stages may be in flight, 4 + na
-    // copies each), refill the slot that stage st - 1 used, compute
-#pragma unroll
-    for (int st = 0; st < S - 1; ++st)
-        if (st < NS) issue(st, st);
-    int slot = 0, prev = S - 1;
+    // ---- the ring: at stage st, wait until it has landed, refill the other slot, which stage
+    // st - 1 used, compute
+    issue(0, 0);
 #pragma unroll 1
     for (int st = 0; st < NS; ++st) {
-        static_assert(S == 2 || S == 3, "wait counts");
-        if (S == 3 && st + 1 < NS) ring_wait_sel<4, 5, 6, 7, 8>(na);
-        else ring_wait<0>();
+        const int slot = st & 1;
+        ring_wait<0>();
         if constexpr (ST != SWQ_F32) {
             // the scale words have landed (they are older than the ring): one wait for them
             // here, not one in every pass (as in pf_gemm_dma)
@@ -1283,12 +1240,10 @@ __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
                     for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bi.s[j][i]));
             }
         }
-        if (st + S - 1 < NS) issue(prev, st + S - 1);
+        if (st + 1 < NS) issue(slot ^ 1, st + 1);
         // (group counts are even, so a short stage of four has two)
         if (GPS == 2 || (st + 1) * GPS <= NG) compute(std::integral_constant<int, GPS>{}, slot, st);
         else compute(std::integral_constant<int, 2>{}, slot, st);
-        prev = slot;
-        slot = slot + 1 == S ? 0 : slot + 1;
     }
 
     if (active) {
@@ -1880,14 +1835,13 @@ int dma_waves(int bits, int npl) { return (bits == 8 && npl == 2) || (bits == 4 
 template <int BITS, int NPL, int EPI>
 void launch_dma_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
     constexpr int W = (BITS == 8 && NPL == 2) || (BITS == 4 && NPL == 1) ? 4 : 8;
-    constexpr int DA = 2, DB = DA + 1;
     const dim3 th(64 * W);
     if (stype == SWQ_F16)
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F16, NPL, EPI, DA, DB, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F16, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
     else if (stype == SWQ_BF16)
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_BF16, NPL, EPI, DA, DB, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_BF16, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
     else
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F32, NPL, EPI, DA, DB, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F32, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
 }
 
 template <int NPL, int EPI>
@@ -1898,18 +1852,12 @@ int launch_dma(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream_
     return launch_status();
 }
 
-// Ring stages of the thin GEMM: two, 43 to 68 KB of LDS and two or three
-// workgroups per CU; three stages measured 36 against 34 us for gate/up and 37
-// against 25 us for down (16 tokens, 256 experts top-8, 4-bit).
-constexpr int kThinStages = 2;
-
 template <int BITS, int NPL, int EPI>
 void launch_thin_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
-    constexpr int D = kThinStages;
     const dim3 g(blocks), th(kPfThreads);
-    if (stype == SWQ_F16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F16, NPL, EPI, D>), g, th, 0, s, a);
-    else if (stype == SWQ_BF16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_BF16, NPL, EPI, D>), g, th, 0, s, a);
-    else hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F32, NPL, EPI, D>), g, th, 0, s, a);
+    if (stype == SWQ_F16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F16, NPL, EPI>), g, th, 0, s, a);
+    else if (stype == SWQ_BF16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_BF16, NPL, EPI>), g, th, 0, s, a);
+    else hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F32, NPL, EPI>), g, th, 0, s, a);
 }
 
 // The thin GEMM over the tile table; sets the column steps and the grid of `a`.
