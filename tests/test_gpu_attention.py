@@ -142,6 +142,38 @@ def test_split_edges(H, KVH, hd, rot, position):
     assert torch.isnan(gk[position + 1:]).all() and np.array_equal(gk[:position].cpu().numpy(), ck)
 
 
+@pytest.mark.parametrize("H,KVH,hd,position", [(32, 8, 128, 33000), (16, 2, 256, 33000), (8, 8, 64, 8200)])
+def test_long_sums_against_64_bits(H, KVH, hd, position):
+    """A split's value sums stay as exact over hundreds of positions as over one tile's.  A chain of m
+    equal steps rounds by about 3.4e-8 (2^-24 / sqrt(3)) of its partial sums at each, 3.4e-8 *
+    sqrt(m / 2) of the result: blocks of 16 and 16 steps of two of them 1e-7 each, with the scores'
+    and the merge's roundings 1.9e-7 measured; one chain of a split's 516 positions 5e-7 (4.3e-7
+    measured).  Bar: 3e-7 relative 2-norm."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(position + hd)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    qw, kw, eps = 1 + 0.1 * r(hd), 1 + 0.1 * r(hd), 1e-6
+    blk = AttentionGPU(H, KVH, hd, 0, 1e7, eps, position + 1, qw, kw)
+    cache, ws = blk.new_cache(), blk.new_workspace()
+    ck, cv = blk.cache_views(cache)
+    ck[:position].normal_(0.0, 0.5, generator=g)
+    cv[:position].normal_(generator=g)
+    q, k, v = r(H, 2, hd), r(KVH, hd), r(KVH, hd)
+    print(f"H {H} KVH {KVH} hd {hd} position {position}", flush=True)
+    out = blk.step(q.reshape(-1), k.reshape(-1), v.reshape(-1), cache, ws, position)
+    norm = lambda x, w: x / (x.pow(2).mean(-1, keepdim=True) + eps).sqrt() * w.double()  # noqa: E731
+    qn = norm(q[:, 0].double(), qw)
+    ck[position].copy_(norm(k.double(), kw).float())
+    want = []
+    for h in range(H):
+        p = ((ck[:, h * KVH // H].double() @ qn[h]) / hd ** 0.5).softmax(0)
+        want.append(p @ cv[:, h * KVH // H].double() * torch.sigmoid(q[h, 1].double()))
+    want = torch.stack(want).reshape(-1)
+    err = float((out.double() - want).norm() / want.norm())
+    print(f"  error {err:.2e}", flush=True)
+    assert err < 3e-7, err
+
+
 def test_tiny_q4_model_entirely_on_the_device_matches_mlx():
     import torch
     from safetensors.numpy import load_file
