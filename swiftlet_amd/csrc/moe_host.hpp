@@ -172,14 +172,12 @@ inline size_t grouped_ws_base(const FusedLayout &f) { return align256(f.total); 
 //   256 experts top-8 (3.1 M
 //   codes a pair)                58/55  65/55  72/58  78/59  103/68  135/79
 //   512 experts top-10           71/61  79/63  89/67  95/71  126/84  170/98
-// Its bias term takes b - 16 s as two bf16 (16 significant bits): whole for f16
-// and bf16 scales, whose sum fits them where b is within a factor of 32 (f16) or
-// 256 (bf16) of 16 s, as quantisers place it; not for f32 ones (1e-5 of one
-// product).  f32 scales on any matrix, f32 activations and 8-bit experts stay with
-// the three launches, which keep scales, x and h in 32 bits there (5e-7 relative;
-// the grouped path splits x and h to 16 significant bits, 5.6e-6), though it would
-// be the faster one at 16 tokens (8-bit 121/104, f32 scales 133/119; at 5 tokens
-// f32 scales 56/69).
+// Its bias term takes b - 16 s in 24 significant bits, which hold all that f16 and
+// bf16 scales can make of it (exponents up to 13 apart) but not f32 ones.  f32
+// scales on any matrix, f32 activations and 8-bit experts stay with the three
+// launches, which keep scales, x and h in 32 bits there (5e-7 relative; the grouped
+// path splits x and h to 16 significant bits, 5.6e-6), though it would be the faster
+// one at 16 tokens (8-bit 121/104, f32 scales 133/119; f32 scales at five 56/69).
 constexpr int kGroupedMinBatch = 5;
 inline bool grouped_pays(const swq_moe_layer *l, int x_dtype, int batch) {
     if (x_dtype != SWQ_BF16 || l->gate.bits != 4 || l->down.bits != 4) return false;

@@ -252,18 +252,34 @@ struct BiasRaw {
     uint32_t b[2][8], s[2][8];
 };
 
+// The parts of b' = b - 16 s (8-bit codes: b) in the bias term: bf16 hi + mid, 16 significant
+// bits, which hold what bf16 scales give unless b is over 256 times 16 s or under a 256th of it,
+// and f16 ones within a factor of 32 (an affine quantiser that keeps zero exact puts |b| at 7.5 s
+// or more); and in the tiles of at most 16 rows, which wide decode batches take too, a third part
+// for whatever 24 bits hold.  Eight tokens, 256 experts top-8, f16 scales, error against 64 bits
+// with two parts / three / the three decode launches: |b| near 0.01 s 1.1e-6 / 1.6e-7 / 2.0e-7,
+// near 750 s 3.0e-6 / 2.3e-6 / 2.4e-6, near 7.5 s 2.6e-6 either way / 3.3e-6; the layer's time
+// 84.1 / 84.2 us at 16 tokens.  In the 64-row tiles it would cost 1% of the time.
+template <int MT>
+struct BiasPlanes {
+    static constexpr bool kLow = MT == 1;
+    static __device__ __forceinline__ void split(const float (&v)[8], u32x4_t &hi, u32x4_t &mid, u32x4_t &lo) {
+        if constexpr (kLow) split8x3(v, hi, mid, lo);
+        else split8(v, hi, mid);
+    }
+};
+
 // The bias term sum_g b'[n,g] X_g[m] over the block's groups below ge, on the
-// group axis, added to acc.  b' is exact as bf16 hi + lo (an fp16 bias less
-// 16 fp16 scales); X_g as hi + mid + lo; the five products above 2^-24
-// relative are accumulated.  xrow[mt]: the group sums of this lane's A row
-// (16 mt + n); entries up to g0 + 31 are readable.
+// group axis, added to acc.  b' as BiasPlanes splits it, X_g as hi + mid + lo;
+// the products above 2^-24 relative are accumulated.  xrow[mt]: the group sums
+// of this lane's A row (16 mt + n); entries up to g0 + 31 are readable.
 template <int BITS, int ST, int MT>
 __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<ST> &r,
                                            const float *const (&xrow)[MT], int g0, int ge, int rows, int kg) {
     float xv[MT][8];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) load_sums8(xrow[mt], g0 + 8 * kg, ge, xv[mt]);
-    u32x4_t bh[2], bl[2];
+    u32x4_t bh[2], bm[2], bl[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         float v[8];
@@ -273,7 +289,7 @@ __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<
             if constexpr (BITS == 4) bp = fmaf(-16.f, scale_of<ST>(r.s[j][i]), bp);
             v[i] = g0 + 8 * kg + i < ge ? bp : 0.f;
         }
-        split8(v, bh[j], bl[j]);
+        BiasPlanes<MT>::split(v, bh[j], bm[j], bl[j]);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -282,10 +298,11 @@ __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<
         split8x3(xv[mt], xh, xm, xl);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
+            if constexpr (BiasPlanes<MT>::kLow) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
             acc[mt][j] = mfma(xl, bh[j], acc[mt][j]);
-            acc[mt][j] = mfma(xm, bl[j], acc[mt][j]);
+            acc[mt][j] = mfma(xm, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bh[j], acc[mt][j]);
-            acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
+            acc[mt][j] = mfma(xh, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xh, bh[j], acc[mt][j]);
         }
     }
@@ -327,7 +344,7 @@ __device__ __forceinline__ void load_bias_bs(BiasBS<ST> &bi, const uint8_t *cons
 template <int BITS, int ST, int MT>
 __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS<ST> &bi, const float (&xv)[MT][8],
                                              int NG, int rows, int kg) {
-    u32x4_t bh[2], bl[2];
+    u32x4_t bh[2], bm[2], bl[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         float v[8];
@@ -345,7 +362,7 @@ __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS
             if constexpr (BITS == 4) bp = fmaf(-16.f, scale_of<ST>(rs), bp);
             v[i] = 8 * kg + i < NG ? bp : 0.f;
         }
-        split8(v, bh[j], bl[j]);
+        BiasPlanes<MT>::split(v, bh[j], bm[j], bl[j]);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -357,10 +374,11 @@ __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS
         split8x3(x, xh, xm, xl);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
+            if constexpr (BiasPlanes<MT>::kLow) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
             acc[mt][j] = mfma(xl, bh[j], acc[mt][j]);
-            acc[mt][j] = mfma(xm, bl[j], acc[mt][j]);
+            acc[mt][j] = mfma(xm, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bh[j], acc[mt][j]);
-            acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
+            acc[mt][j] = mfma(xh, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xh, bh[j], acc[mt][j]);
         }
     }
@@ -1061,7 +1079,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 
 constexpr int kThinRows = 16;
 
-// pf_gemm_dma for tiles of at most kThinRows rows, bit for bit.  With few rows
+// pf_gemm_dma for tiles of at most kThinRows rows, bit for bit where b - 16 s has 16 significant
+// bits (see BiasPlanes).  With few rows
 // the codes are the work, and a ring of single 64-input groups reads them in
 // 32-byte pieces and pays a barrier and an LDS round trip per group.  Here a
 // ring stage is 128 bytes of every code row, whole cache lines (four groups of

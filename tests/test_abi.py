@@ -89,8 +89,8 @@ EXPERTS = ("gate", "up", "down", "shared_gate", "shared_up", "shared_down")
 @pytest.mark.parametrize("wide", [("router",), EXPERTS, ("router",) + EXPERTS], ids=["router", "experts", "all"])
 def test_f32_scales_keep_the_three_launches(lib, wide):
     """A wide batch is regrouped by expert only where every scale has two bytes (the regrouped
-    contraction holds b - 16 s in 16 significant bits): with f32 scales the workspace is that of
-    the three launches, as it is for 8-bit experts."""
+    contraction holds b - 16 s in 24 significant bits, all that those make of it): with f32 scales
+    the workspace is that of the three launches, as it is for 8-bit experts."""
     L = layer()
     staged = lib.swq_moe_decode_workspace_bytes(ctypes.byref(layer(bits=8)), 8)
     assert lib.swq_moe_decode_workspace_bytes(ctypes.byref(L), 8) > staged

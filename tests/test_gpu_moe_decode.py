@@ -438,25 +438,39 @@ def test_wide_batches_take_the_grouped_path(name, batch, x_dtype, grouped):
 def _dense64(lin, e=0):
     """Expert e of a 4- or 8-bit GPULinear in 64 bits, on the device."""
     import torch
+    from swiftlet_amd import _lib
+    dt = {_lib.SWQ_F32: torch.float32, _lib.SWQ_F16: torch.float16, _lib.SWQ_BF16: torch.bfloat16}[lin.scales_type]
     per = 32 // lin.bits
     words = lin.w.view(torch.int32)[e * lin.expert_stride_w // 4:][:lin.out_dim * lin.in_dim // per].long()
     codes = (words.unsqueeze(1) >> (lin.bits * torch.arange(per, device=words.device))) & ((1 << lin.bits) - 1)
     n = lin.out_dim * lin.in_dim // lin.group_size
-    s, b = (t.view(torch.float32)[e * lin.expert_stride_sb // 4:][:n].double().unsqueeze(1) for t in (lin.scales, lin.biases))
+    s, b = (t.view(dt)[e * lin.expert_stride_sb // dt.itemsize:][:n].double().unsqueeze(1) for t in (lin.scales, lin.biases))
     return (codes.reshape(n, lin.group_size) * s + b).reshape(lin.out_dim, lin.in_dim)
+
+
+def _moe64(gpu, x, ids):
+    """The layer over x in 64 bits, with the picks given."""
+    import torch
+    xd = x.double()
+    ffn = lambda v, g, u, d: d @ (torch.nn.functional.silu(g @ v) * (u @ v))  # noqa: E731
+    top = (xd @ _dense64(gpu.router).t()).softmax(1).gather(1, ids.long())
+    top = top / top.sum(1, keepdim=True)
+    out = torch.stack([sum(top[t, k] * ffn(xd[t], *(_dense64(m, int(ids[t, k])) for m in (gpu.gate, gpu.up, gpu.down)))
+                           for k in range(gpu.top_k)) for t in range(x.shape[0])])
+    shared = [_dense64(m) for m in (gpu.shared_gate, gpu.shared_up, gpu.shared_down)]
+    return out + torch.sigmoid(xd @ _dense64(gpu.shared_expert_gate).t()) * torch.stack([ffn(v, *shared) for v in xd])
 
 
 @pytest.mark.parametrize("name,batch", [("qwen3.6-35b-a3b-q4", 8), ("qwen3-next-80b-a3b-q4", 5)])
 def test_wide_batch_of_f32_scales(name, batch):
     """Scales and biases that need all of their 32 bits, in a batch wide enough for the grouped
     path with 2-byte ones: the three launches' bits, and within 1e-5 of 64 bits (the dot products
-    split h to 16 significant bits, 3.5e-6; a bias term in 16 bits would add 1e-5 per product)."""
+    split h to 16 significant bits, 3.5e-6)."""
     import torch
     shape = synth.SHAPES[name]
     gpu = helpers.widen_layer(moe.synth_layer(shape, helpers.SEED, 0))
     g = torch.Generator(device="cuda").manual_seed(7)
-    mats = [gpu.router, gpu.gate, gpu.up, gpu.down, gpu.shared_gate, gpu.shared_up, gpu.shared_down]
-    for m in mats:
+    for m in (gpu.router, gpu.gate, gpu.up, gpu.down, gpu.shared_gate, gpu.shared_up, gpu.shared_down):
         for t in (m.scales, m.biases):
             f = t.view(torch.float32)
             f.mul_(1 + 0.01 * torch.rand(f.shape, generator=g, device="cuda"))
@@ -467,16 +481,39 @@ def test_wide_batch_of_f32_scales(name, batch):
     out, ids, w = gpu.decode(x, ws=ws)
     torch.cuda.synchronize()
     assert torch.equal(out, staged) and torch.equal(ids, i_s) and torch.equal(w, w_s)
-    xd = x.double()
-    probs = (xd @ _dense64(gpu.router).t()).softmax(1)
-    top = probs.gather(1, ids.long())
-    top = top / top.sum(1, keepdim=True)
-    ffn = lambda v, gm, um, dm: dm @ (torch.nn.functional.silu(gm @ v) * (um @ v))  # noqa: E731
-    seg = gpu.shared_expert_gate
-    want = torch.stack([sum(top[t, k] * ffn(xd[t], *(_dense64(m, int(ids[t, k])) for m in mats[1:4]))
-                            for k in range(shape.top_k)) for t in range(batch)])
-    gate = torch.sigmoid(xd @ _dense64(seg).t())
-    want += gate * torch.stack([ffn(xd[t], *(_dense64(m) for m in mats[4:])) for t in range(batch)])
-    err = R.rel_l2(out.double().cpu().numpy(), want.cpu().numpy())
+    err = R.rel_l2(out.double().cpu().numpy(), _moe64(gpu, x, ids).cpu().numpy())
     print(f"  rel L2 {err:.2e} of 64 bits", flush=True)
     assert err < 1e-5, err
+
+
+@pytest.mark.parametrize("ratio", [0.01, 0.5, 750.0])
+def test_wide_batch_of_any_bias(ratio):
+    """f16 biases far from 16 s, |b| about `ratio` times s: b - 16 s then needs more than 16
+    significant bits, and the grouped path keeps them.  The three launches on the same input are
+    the yardstick (they use b and s as they are): the grouped path is no further from 64 bits than
+    they are, but for a third of their error or 1e-7 (the order of 32-bit sums).  With 16 bits it
+    was 5 times as far for 0.01."""
+    import torch
+    from swiftlet_amd.engine import GPULinear
+    shape = synth.SHAPES["qwen3.6-35b-a3b-q4"]
+    gpu = moe.synth_layer(shape, helpers.SEED, 0)
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def move(m):
+        s = m.scales.view(torch.float16).float() * (1.0 if m.bits == 4 else 17.0)  # 4-bit and 8-bit codes alike
+        b = (ratio * s * torch.randn(s.shape, generator=g, device="cuda")).half().view(torch.uint8)
+        return GPULinear(m.w, m.scales, b, m.out_dim, m.in_dim, m.group_size, m.bits, m.scales_type,
+                         expert_stride_w=m.expert_stride_w, expert_stride_sb=m.expert_stride_sb, num_experts=m.num_experts)
+    far = moe.MoELayerGPU(*(move(m) for m in (gpu.router, gpu.gate, gpu.up, gpu.down, gpu.shared_gate, gpu.shared_up,
+                                              gpu.shared_down, gpu.shared_expert_gate)), top_k=shape.top_k)
+    x = helpers.bf16_bits_to_torch(synth.activations_bf16(helpers.SEED + 23, 8, shape.hidden))
+    print(f"biases of {ratio} scales", flush=True)
+    ws = far.new_workspace(8)
+    staged, i_s, _ = far.decode(x, ws=ws, path="staged")
+    out, ids, _ = far.decode(x, ws=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(ids, i_s) and not torch.equal(out, staged)
+    want = _moe64(far, x, ids).cpu().numpy()
+    grouped, three = (R.rel_l2(t.double().cpu().numpy(), want) for t in (out, staged))
+    print(f"  grouped {grouped:.2e}, three launches {three:.2e}", flush=True)
+    assert grouped < max(4 / 3 * three, three + 1e-7), (grouped, three)
