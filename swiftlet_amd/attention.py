@@ -11,8 +11,7 @@ import ctypes
 
 from . import _lib
 from ._lib import AttentionLayer, check
-from .engine import (ENGINE_LAUNCHES, DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch,
-                     replaced)
+from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch, own_launches
 
 
 class AttentionGPU:
@@ -80,10 +79,10 @@ class AttentionGPU:
         RMSNorm runs inside that launch), the step, o_proj.  One native call,
         or the launches one by one where `step` or one of the engine's has been
         overridden."""
-        if _elsewhere(stream):
+        if stream is not None and _elsewhere(stream):
             with _torch().cuda.stream(stream):
                 return AttentionGPU.forward_token(self, engine, x, cache, ws, position, norm_weight, eps)
-        if replaced(engine, ENGINE_LAUNCHES) or replaced(self, _STEP):
+        if not own_launches(engine, self.step, _OWN_STEP):
             return self._forward_launches(engine, x, cache, ws, position, norm_weight, eps, stream)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         pq, pk, pv = self.projections
@@ -108,7 +107,7 @@ class AttentionGPU:
         return r
 
 
-_STEP = (("step", AttentionGPU.step),)
+_OWN_STEP = AttentionGPU.step
 
 
 def attention_from_checkpoint(ckpt, layer: int, config: dict, max_positions: int = 4096, device="cuda",

@@ -10,8 +10,7 @@ import ctypes
 
 from . import _lib
 from ._lib import SWQ_DELTA_INTERLEAVED, SWQ_DELTA_SPLIT, DeltaNetLayer, check
-from .engine import (ENGINE_LAUNCHES, DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch,
-                     replaced)
+from .engine import DescArray, GPULinear, HipEngine, _elsewhere, _norm_arg, _stream_handle, _torch, own_launches
 
 
 class DeltaNetGPU:
@@ -85,10 +84,10 @@ class DeltaNetGPU:
         input RMSNorm runs inside that launch), the step, out_proj.  One native
         call, or the launches one by one where `step` or one of the engine's
         has been overridden."""
-        if _elsewhere(stream):
+        if stream is not None and _elsewhere(stream):
             with _torch().cuda.stream(stream):
                 return DeltaNetGPU.forward_token(self, engine, x, state, position, norm_weight, eps)
-        if replaced(engine, ENGINE_LAUNCHES) or replaced(self, _STEP):
+        if not own_launches(engine, self.step, _OWN_STEP):
             return self._forward_launches(engine, x, state, position, norm_weight, eps, stream)
         empty, f32, dev = _torch().empty, _torch().float32, x.device
         scratch = empty(self._scratch, dtype=f32, device=dev)
@@ -115,7 +114,7 @@ class DeltaNetGPU:
         return r
 
 
-_STEP = (("step", DeltaNetGPU.step),)
+_OWN_STEP = DeltaNetGPU.step
 
 
 def deltanet_from_checkpoint(ckpt, layer: int, config: dict, device="cuda", stream=None) -> DeltaNetGPU:

@@ -278,14 +278,14 @@ class HipEngine:
         return out
 
 
-# the launches that a block's forward_token makes in one native call instead
-ENGINE_LAUNCHES = (("encode_gemv", HipEngine.encode_gemv), ("encode_gemv_multi", HipEngine.encode_gemv_multi))
+_OWN_GEMV, _OWN_MULTI = HipEngine.encode_gemv, HipEngine.encode_gemv_multi
 
 
-def replaced(obj, methods) -> bool:
-    """Whether `obj` has another function than its class's own under one of these names: a
-    subclass's, an instance's, or one put in place of the class's."""
-    for name, own in methods:
-        if getattr(getattr(obj, name, None), "__func__", None) is not own:
-            return True
-    return False
+def own_launches(engine, step, own_step) -> bool:
+    """Whether the launches that a block's forward_token makes in one native call are the classes'
+    own: not a subclass's, an instance's, or ones put in place of the classes'."""
+    try:
+        return (engine.encode_gemv.__func__ is _OWN_GEMV and engine.encode_gemv_multi.__func__ is _OWN_MULTI
+                and step.__func__ is own_step)
+    except AttributeError:
+        return False
