@@ -459,15 +459,19 @@ int swq_moe_workspace_status(void *ws, size_t ws_bytes, int clear, void *stream)
  * device.  Batch 1 runs as one launch (router, softmax, top-k with ties to the
  * lower expert id, renormalisation, routed SwiGLU experts, down projections,
  * sigmoid-gated shared expert and the weighted combine; its stages hand data
- * to each other through the workspace).  Batches run as three launches:
+ * to each other through the workspace), batches of 2 and 4 too where batch *
+ * top_k <= 32.  Others run as three launches:
  *   1. router GEMV + shared-gate GEMV + shared gate/up SwiGLU;
  *   2. top-k per token, the distinct experts, their gate/up SwiGLU rows for
  *      all their tokens, indexed by the device-resident ids;
  *   3. down projections + weighted combine + sigmoid-gated shared expert;
- * or, from five tokens on with bf16 x and 4-bit experts that are large enough,
- * as swq_moe_prefill's launches (the pairs sorted by expert, matrix cores), if
- * the prefill takes the layer, out is 16-byte aligned and the workspace holds
- * swq_moe_decode_workspace_bytes(layer, batch).
+ * or, from five tokens on with bf16 x, 4-bit experts that are large enough and
+ * no f32 scales, as swq_moe_prefill's launches (the pairs sorted by expert,
+ * matrix cores), if the prefill takes the layer, out is 16-byte aligned and the
+ * workspace holds swq_moe_decode_workspace_bytes(layer, batch).  The one launch
+ * gives the three launches' bits; the prefill's launches give others, no further
+ * from exact (3e-6 relative either way), so a token's last bits can differ
+ * between a batch of up to four and a wider one.
  * x: [batch, hidden] of x_dtype (SWQ_F32 / SWQ_BF16).  out: [batch, hidden]
  * of out_dtype (SWQ_F32 / SWQ_BF16).  topk_ids [batch, top_k] int32 and
  * topk_weights [batch, top_k] f32 receive the routing (either may be NULL).
@@ -530,9 +534,10 @@ size_t swq_moe_prefill_workspace_bytes(const swq_moe_layer *layer, int tokens);
  * on its own exactly as in swq_moe_decode, with the (token, expert) pairs
  * grouped by expert so each expert's weights are contracted against all of
  * its tokens at once on the bf16 matrix cores (codes exact in bf16, fp32
- * accumulation, per-group scales applied in fp32).  Five launches: router
- * GEMM; top-k + grouping; gate/up + SwiGLU; down; weighted combine in pick
- * order, then the sigmoid-gated shared expert.
+ * accumulation, per-group scales applied in fp32).  Six launches: router GEMM;
+ * top-k; grouping (two launches above 8,192 pairs); gate/up + SwiGLU; down;
+ * weighted combine in pick order, then the sigmoid-gated shared expert.  A
+ * workspace made for some number of tokens serves fewer too.
  * Formats: 4/8-bit codes with group 64 for the router, routed and shared
  * matrices; in_dim a multiple of 128 and at most 4096; the shared gate/up and
  * down matrices with the routed ones' bit widths.  Others: SWQ_ERR_LIMIT.

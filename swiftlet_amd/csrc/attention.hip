@@ -487,7 +487,10 @@ size_t half_cache(const swq_attention_layer *l) {
 // round trip, so a short context is fastest spread thin), else that many workgroups, each
 // walking its positions two tiles a step.  Step + merge at 33,001 positions and 2 kv heads:
 // 256 workgroups 42.7 us, 512 38.5, 1,024 41.0; at 4,096 13.5, 13.7, 13.6; at 1,000 the
-// 64-position workgroups of four waves took 15.0, one tile each 10.2.
+// 64-position workgroups of four waves took 15.0, one tile each 10.2.  Past a whole step the last
+// one is mostly padding, which costs up to a fifth: at 2 kv heads 4,096 / 4,097 positions 11.8 /
+// 13.4 us, 8,192 / 8,193 14.5 / 17.2, 16,384 / 16,385 19.4 / 22.8, 32,768 / 33,001 32.4 / 38.3
+// (64-position chunks: 18.5 / 17.9, 23.0 / 30.6, 40.4 / 46.3, 74.4 / 81.5).
 struct AttnPlan {
     int per, splits, tiles;
 };

@@ -1,22 +1,25 @@
 // Ragged MoE prefill on gfx950: the layer of QwenCPUModel.moeForward
 // (QwenCPUModel.swift:500-569) applied to S tokens at once.  The (token,
 // expert) pairs are grouped by expert, so each expert's weights are read once
-// per tile of up to 64 of its tokens and contracted on the bf16 matrix cores.
+// per tile of up to 64 of its tokens (16 where the experts see few) and
+// contracted on the bf16 matrix cores.
 // The grouping follows mlx's _gather_sort / gather_qmm / _scatter_unsort
 // (switch_layers.py:12-24, 75-90, 176-199); the arithmetic follows the CPU
 // path, which loops the same per-token computation (QwenCPUModel.swift:544-567).
 //
 // Launches, all on the caller's stream:
-//   1. router GEMM: partial logits [slice][T, E], 16-token tiles x K slices
-//      of 4 groups; its first column block also writes x in the layout
-//      gate/up reads (bf16 planes) and the group sums of x;
+//   1. router GEMM: partial logits [slice][T, E], tiles of 16 tokens (32 from
+//      1,024 on) x K slices of 4 groups; its first column block also writes x
+//      in the layout gate/up reads (bf16 planes) and the group sums of x;
 //   2. route: softmax, top-k (ties to the lower id), renormalisation and
 //      the shared-expert gate logit per token;
-//   2b. group: one workgroup of 1024 threads counts the pairs per expert and
-//      builds the sorted pair order and the table of 64-row tiles (routed
-//      experts, then the shared expert over all tokens);
+//   2b. group: counts the pairs per expert and builds the sorted pair order and
+//      the table of 64-row or 16-row tiles (routed experts, then the shared
+//      expert over all tokens); one workgroup of 1024 threads, above 8,192
+//      pairs two launches of 32 workgroups;
 //   3. gate/up GEMM over the tile table with the SwiGLU epilogue: h in
-//      sorted pair order, as bf16 hi + lo planes;
+//      sorted pair order, as bf16 hi + lo planes (pf_gemm_dma for 64-row
+//      tiles, pf_gemm_thin for 16-row ones; so too 4.);
 //   4. down GEMM over the same tiles: y rows (f32) in sorted pair order;
 //   5. combine: out[t] = sum_k w_tk y[pos(t,k)] in pick order, then
 //      + sigmoid(sg_t) y_shared[t] (QwenCPUModel.swift:556, :566).
@@ -32,7 +35,7 @@
 // or split into bf16 hi + lo (fp32 inputs, the SwiGLU output), one MFMA per
 // part.  Every product is exact and accumulates in fp32, the scale applies
 // per group in fp32, and the bias term is one more MFMA chain over the group
-// axis with both factors split hi + lo.
+// axis with X_g in three bf16 parts and b' in two or three (BiasPlanes).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1686,7 +1689,9 @@ int router_kslices(int H) { return (H / kGroupK + kBlockG - 1) / kBlockG; }
 //   256 experts top-8, 4-bit  84/74 120/103 135/121 149/138 159/153 194/212
 //   256 experts top-8, 8-bit 112/103 155/131 185/166 200/185 213/202 247/276
 //   512 experts top-10, 4-bit 113/98 161/139 196/171 221/200 237/223 309/316
-// (f32 x at 256 tokens, 4-bit: 165/170.)
+// (f32 x at 256 tokens, 4-bit: 165/170.)  The rule has no code width: with 8-bit codes and bf16 x
+// gate/up alone is slower in 16-row tiles at 16 tokens (56.4/58.8; at 77 109.5/103.7), down's gain
+// is the larger one (39.9/30.5, 80.0/61.0).
 constexpr int kThinAvgRows = 6;
 int most_thin_tokens(const swq_moe_layer *l) { return std::max(kThinRows, kThinAvgRows * l->num_experts / l->top_k); }
 bool thin_tiles(const swq_moe_layer *l, int T) { return T <= most_thin_tokens(l); }
@@ -1846,9 +1851,13 @@ int launch_gemm(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream
 // 113 -> 108.5 us on the 512-token chunk; down at 4 waves loses, 74 -> 79 us
 // there, 261 -> 280 at 4,096 tokens).  8-bit codes with two activation planes:
 // 4 waves.  Activation rings are two groups deep: four workgroups per CU, 16
-// waves, cover the waits better than a third group in the LDS of three does
-// (4-bit gate/up, bf16 x: 106.7 -> 97.8 us at 512 tokens, 322 -> 302 at 4,096;
-// five, with the group sums read at the end instead of held in LDS, spill).
+// waves, cover the waits better than a third group in the LDS of three does,
+// by an amount that goes with the load (4-bit gate/up, bf16 x, us with three /
+// two groups, both in turn: 512 tokens 102.9/102.5 with evenly loaded experts,
+// 100.8/96.7 where some are busier, 105.0/104.3 at a Zipf load; 4,096 tokens
+// 314.7/301.0 and 310.3/303.9.  Without the branch per wait count, which deeper
+// rings needed, 100.0, 95.4, 103.2, 297 and 298).  Five, with the group sums read
+// at the end instead of held in LDS, spill.
 int dma_waves(int bits, int npl) { return (bits == 8 && npl == 2) || (bits == 4 && npl == 1) ? 4 : 8; }
 
 template <int BITS, int NPL, int EPI>

@@ -87,8 +87,10 @@ class MoELayerGPU:
         """One decode step for x [B, H] (bf16 or f32 device tensor).
 
         ``path``: "auto" (swq_moe_decode: one launch when the layer and batch
-        allow, else three), "staged" (the three launches) or "fused" (the
-        single launch; raises SwqError LIMIT when it cannot take the call).
+        allow, the prefill's launches for five tokens or more of bf16 x with
+        4-bit experts and 2-byte scales, else three), "staged" (the three
+        launches) or "fused" (the single launch; raises SwqError LIMIT when it
+        cannot take the call).
         Without ``ws`` the call makes a workspace and reads its stall record
         afterwards (blocking; SwqError STALLED if a bounded wait ran out);
         with ``ws`` the caller reads it with workspace_status.

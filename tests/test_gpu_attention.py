@@ -8,9 +8,9 @@ over max abs value); the cache rows the step appends within the same bound
 (normalised, rotated k; v bit-exact).  Cases: the tiny model's attention
 shape (hd 16, 4 heads over 2 kv heads, 4 rotary dims) token by token; the
 35B / 80B shape (16 heads over 2 kv heads, hd 256, 64 rotary dims, theta
-1e7) token by token across the 64-position split boundary, and single steps
-at positions 1000 and 5000 over a random cache (several splits, chunks
-above the minimum); and the reference's tiny 4-bit qwen3_next model run
+1e7) token by token over five splits of 16 positions, and single steps
+at positions 1000 and 5000 over a random cache (splits of one tile, and of
+more); and the reference's tiny 4-bit qwen3_next model run
 entirely on the device — embedding rows, every norm, DeltaNet and attention
 block (input norm fused into the projections' launch), MoE block and the
 lm_head — against mlx's logits (2e-3,
