@@ -35,7 +35,7 @@
 // or split into bf16 hi + lo (fp32 inputs, the SwiGLU output), one MFMA per
 // part.  Every product is exact and accumulates in fp32, the scale applies
 // per group in fp32, and the bias term is one more MFMA chain over the group
-// axis with X_g in three bf16 parts and b' in two or three (BiasPlanes).
+// axis with X_g in three bf16 parts and b' in two or three (bias_parts).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -258,25 +258,24 @@ struct BiasRaw {
 // The parts of b' = b - 16 s (8-bit codes: b) in the bias term: bf16 hi + mid, 16 significant
 // bits, which hold what bf16 scales give unless b is over 256 times 16 s or under a 256th of it,
 // and f16 ones within a factor of 32 (an affine quantiser that keeps zero exact puts |b| at 7.5 s
-// or more); and in the tiles of at most 16 rows, which wide decode batches take too, a third part
-// for whatever 24 bits hold.  Eight tokens, 256 experts top-8, f16 scales, error against 64 bits
-// with two parts / three / the three decode launches: |b| near 0.01 s 1.1e-6 / 1.6e-7 / 2.0e-7,
-// near 750 s 3.0e-6 / 2.3e-6 / 2.4e-6, near 7.5 s 2.6e-6 either way / 3.3e-6; the layer's time
-// 84.1 / 84.2 us at 16 tokens.  In the 64-row tiles it would cost 1% of the time.
-template <int MT>
-struct BiasPlanes {
-    static constexpr bool kLow = MT == 1;
-    static __device__ __forceinline__ void split(const float (&v)[8], u32x4_t &hi, u32x4_t &mid, u32x4_t &lo) {
-        if constexpr (kLow) split8x3(v, hi, mid, lo);
-        else split8(v, hi, mid);
-    }
-};
+// or more); and with WHOLE a third part for whatever 24 bits hold: decode batches, whose other
+// launches use b and s as they are.  Eight tokens, 256 experts top-8, f16 scales, error against
+// 64 bits with two parts / three / the three decode launches: |b| near 0.01 s 1.1e-6 / 1.6e-7 /
+// 2.0e-7, near 750 s 3.0e-6 / 2.3e-6 / 2.4e-6, near 7.5 s 2.6e-6 either way / 3.3e-6.  It takes
+// 0.8 us of the 81 of a 16-token layer and would take up to 2% of a prefill with f32 x, which keeps
+// two.  Measured beside it: a flag in the arguments instead of instances of their own, 2.3 us; the
+// parts formed while the second stage comes in, 30 more registers and 3.5 us.
+template <bool WHOLE>
+__device__ __forceinline__ void bias_parts(const float (&v)[8], u32x4_t &hi, u32x4_t &mid, u32x4_t &lo) {
+    if constexpr (WHOLE) split8x3(v, hi, mid, lo);
+    else split8(v, hi, mid);
+}
 
 // The bias term sum_g b'[n,g] X_g[m] over the block's groups below ge, on the
-// group axis, added to acc.  b' as BiasPlanes splits it, X_g as hi + mid + lo;
+// group axis, added to acc.  b' in bias_parts' two or three, X_g as hi + mid + lo;
 // the products above 2^-24 relative are accumulated.  xrow[mt]: the group sums
 // of this lane's A row (16 mt + n); entries up to g0 + 31 are readable.
-template <int BITS, int ST, int MT>
+template <int BITS, int ST, int MT, bool WHOLE>
 __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<ST> &r,
                                            const float *const (&xrow)[MT], int g0, int ge, int rows, int kg) {
     float xv[MT][8];
@@ -292,7 +291,7 @@ __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<
             if constexpr (BITS == 4) bp = fmaf(-16.f, scale_of<ST>(r.s[j][i]), bp);
             v[i] = g0 + 8 * kg + i < ge ? bp : 0.f;
         }
-        BiasPlanes<MT>::split(v, bh[j], bm[j], bl[j]);
+        bias_parts<WHOLE>(v, bh[j], bm[j], bl[j]);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -301,7 +300,7 @@ __device__ __forceinline__ void bias_apply(f32x4_t (&acc)[MT][2], const BiasRaw<
         split8x3(xv[mt], xh, xm, xl);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (BiasPlanes<MT>::kLow) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
+            if constexpr (WHOLE) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
             acc[mt][j] = mfma(xl, bh[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bh[j], acc[mt][j]);
@@ -344,7 +343,7 @@ __device__ __forceinline__ void load_bias_bs(BiasBS<ST> &bi, const uint8_t *cons
 
 // bias_term from preloaded biases/scales and the lane's group sums xv[mt]
 // (NG <= 32).
-template <int BITS, int ST, int MT>
+template <int BITS, int ST, int MT, bool WHOLE = false>
 __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS<ST> &bi, const float (&xv)[MT][8],
                                              int NG, int rows, int kg) {
     u32x4_t bh[2], bm[2], bl[2];
@@ -365,7 +364,7 @@ __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS
             if constexpr (BITS == 4) bp = fmaf(-16.f, scale_of<ST>(rs), bp);
             v[i] = 8 * kg + i < NG ? bp : 0.f;
         }
-        BiasPlanes<MT>::split(v, bh[j], bm[j], bl[j]);
+        bias_parts<WHOLE>(v, bh[j], bm[j], bl[j]);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
@@ -377,7 +376,7 @@ __device__ __forceinline__ void bias_term_bs(f32x4_t (&acc)[MT][2], const BiasBS
         split8x3(x, xh, xm, xl);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (BiasPlanes<MT>::kLow) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
+            if constexpr (WHOLE) acc[mt][j] = mfma(xh, bl[j], acc[mt][j]);
             acc[mt][j] = mfma(xl, bh[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bm[j], acc[mt][j]);
             acc[mt][j] = mfma(xm, bh[j], acc[mt][j]);
@@ -478,7 +477,7 @@ constexpr int kBlockG = 4;  // pf_gemm: K groups staged per round trip
 // columns); see the file comment for the arithmetic.  Rows past the tile
 // (`rows`) are staged from row 0 and never stored: the matrix cores keep rows
 // apart, so they cannot disturb the others.
-template <int BITS, int ST, int SRC, int MT, int EPI, int SUM>
+template <int BITS, int ST, int SRC, int MT, int EPI, int SUM, bool WHOLE>
 __global__ __launch_bounds__(kPfThreads) void pf_gemm(const GemmArgs a) {
     constexpr int ROWS = 16 * MT;
     constexpr int NPL = SRC == kSrcBF16 ? 1 : 2;
@@ -786,7 +785,7 @@ __global__ __launch_bounds__(kPfThreads) void pf_gemm(const GemmArgs a) {
                 braw.b[j][i] = tab(j, 1, g);
                 braw.s[j][i] = tab(j, 0, g);
             }
-        bias_apply<BITS, ST, MT>(acc, braw, xrow, gb, ge, rows, kg);
+        bias_apply<BITS, ST, MT, WHOLE>(acc, braw, xrow, gb, ge, rows, kg);
     }
     epilogue<EPI, MT>(acc, a, col, N, active, row0, rows, nb, s_red, static_cast<int64_t>(blockIdx.y) * a.o_slice);
 }
@@ -1083,7 +1082,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 constexpr int kThinRows = 16;
 
 // pf_gemm_dma for tiles of at most kThinRows rows, bit for bit where b - 16 s has 16 significant
-// bits (see BiasPlanes).  With few rows
+// bits, or with two parts of it (see bias_parts).  With few rows
 // the codes are the work, and a ring of single 64-input groups reads them in
 // 32-byte pieces and pays a barrier and an LDS round trip per group.  Here a
 // ring stage is 128 bytes of every code row, whole cache lines (four groups of
@@ -1100,7 +1099,7 @@ constexpr int kThinRows = 16;
 // waves, 60 and 35 us at 16 tokens; one-wave workgroups, 256-byte row pieces
 // in 32 KB of LDS, 57 and 45; the single-group ring with 16-row activation
 // slots six groups deep, 42 and 26.
-template <int BITS, int ST, int NPL, int EPI>
+template <int BITS, int ST, int NPL, int EPI, bool WHOLE>
 __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
     constexpr int WAVES = 4, GPS = BITS == 4 ? 4 : 2;  // groups per stage
     constexpr int A_GROUP = NPL * kThinRows * 128, A_STAGE = GPS * A_GROUP;
@@ -1273,7 +1272,7 @@ __global__ __launch_bounds__(kPfThreads) void pf_gemm_thin(const GemmArgs a) {
         const float4 x0 = *reinterpret_cast<const float4 *>(xr + 16 * ((2 * kg) ^ x7));
         const float4 x1 = *reinterpret_cast<const float4 *>(xr + 16 * ((2 * kg + 1) ^ x7));
         const float xv[1][8] = {{x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w}};
-        bias_term_bs<BITS, ST, 1>(acc, bi, xv, NG, rows, kg);
+        bias_term_bs<BITS, ST, 1, WHOLE>(acc, bi, xv, NG, rows, kg);
     }
     epilogue<EPI, 1, WAVES>(acc, a, col, N, active, row0, rows, nb, s_red);
 }
@@ -1817,28 +1816,29 @@ int check_prefill_layer(const swq_moe_layer *l, int T) {
     return SWQ_OK;
 }
 
-template <int BITS, int SRC, int MT, int EPI, int SUM>
+template <int BITS, int SRC, int MT, int EPI, int SUM, bool WHOLE>
 void launch_gemm_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
     const dim3 grid(blocks, a.kslices);
     if (stype == SWQ_F16)
-        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_F16, SRC, MT, EPI, SUM>), grid, dim3(kPfThreads), 0, s, a);
+        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_F16, SRC, MT, EPI, SUM, WHOLE>), grid, dim3(kPfThreads), 0, s, a);
     else if (stype == SWQ_BF16)
-        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_BF16, SRC, MT, EPI, SUM>), grid, dim3(kPfThreads), 0, s, a);
-    else
-        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_F32, SRC, MT, EPI, SUM>), grid, dim3(kPfThreads), 0, s, a);
+        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_BF16, SRC, MT, EPI, SUM, WHOLE>), grid, dim3(kPfThreads), 0, s, a);
+    else if constexpr (!WHOLE)  // (no f32 scales in a decode batch)
+        hipLaunchKernelGGL((pf_gemm<BITS, SWQ_F32, SRC, MT, EPI, SUM, WHOLE>), grid, dim3(kPfThreads), 0, s, a);
 }
 
-template <int SRC, int MT, int EPI, int SUM>
+template <int SRC, int MT, int EPI, int SUM, bool WHOLE = false>
 int launch_gemm(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream_t s) {
     if (blocks <= 0) return SWQ_OK;
+    if (WHOLE && lin.scales_type == SWQ_F32) return SWQ_ERR_LIMIT;
     // slices of kBlockG groups cover the rows' groups (an even count), the
     // scale table covers the column block; tiled rows hold one slice
     const int NG = a.K / kGroupK;
     if (a.kgroups != std::min(kBlockG, NG) || a.kslices != (NG + kBlockG - 1) / kBlockG || a.col_block > 128 ||
         a.col_wave != 32 || a.col_op != 16 || (a.kslices > 1 && (a.tiles || EPI != kEpiRows)))
         return SWQ_ERR_INVALID_ARGUMENT;
-    if (lin.bits == 4) launch_gemm_st<4, SRC, MT, EPI, SUM>(lin.scales_type, a, blocks, s);
-    else launch_gemm_st<8, SRC, MT, EPI, SUM>(lin.scales_type, a, blocks, s);
+    if (lin.bits == 4) launch_gemm_st<4, SRC, MT, EPI, SUM, WHOLE>(lin.scales_type, a, blocks, s);
+    else launch_gemm_st<8, SRC, MT, EPI, SUM, WHOLE>(lin.scales_type, a, blocks, s);
     return launch_status();
 }
 
@@ -1880,29 +1880,36 @@ int launch_dma(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream_
     return launch_status();
 }
 
-template <int BITS, int NPL, int EPI>
+template <int BITS, int NPL, int EPI, bool WHOLE>
 void launch_thin_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
     const dim3 g(blocks), th(kPfThreads);
-    if (stype == SWQ_F16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F16, NPL, EPI>), g, th, 0, s, a);
-    else if (stype == SWQ_BF16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_BF16, NPL, EPI>), g, th, 0, s, a);
-    else hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F32, NPL, EPI>), g, th, 0, s, a);
+    if (stype == SWQ_F16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F16, NPL, EPI, WHOLE>), g, th, 0, s, a);
+    else if (stype == SWQ_BF16) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_BF16, NPL, EPI, WHOLE>), g, th, 0, s, a);
+    else if constexpr (!WHOLE) hipLaunchKernelGGL((pf_gemm_thin<BITS, SWQ_F32, NPL, EPI, WHOLE>), g, th, 0, s, a);
 }
 
-// The thin GEMM over the tile table; sets the column steps and the grid of `a`.
+// The thin GEMM over the tile table; sets the column steps and the grid of `a`.  whole: a decode
+// batch (4-bit codes, 2-byte scales), with every bit of the bias (bias_parts).
 template <int NPL, int EPI>
-int launch_thin(const swq_qlinear &lin, GemmArgs &a, int max_tiles, int N, hipStream_t s) {
+int launch_thin(const swq_qlinear &lin, GemmArgs &a, int max_tiles, int N, bool whole, hipStream_t s) {
     a.col_block = 4 * a.col_wave;
     a.nblk = (N + a.col_block - 1) / a.col_block;
     const int blocks = gemm_blocks(max_tiles, a.nblk);
     if (blocks <= 0) return SWQ_OK;
-    if (lin.bits == 4) launch_thin_st<4, NPL, EPI>(lin.scales_type, a, blocks, s);
-    else launch_thin_st<8, NPL, EPI>(lin.scales_type, a, blocks, s);
+    if (whole) {
+        if (lin.bits != 4 || lin.scales_type == SWQ_F32) return SWQ_ERR_LIMIT;
+        launch_thin_st<4, NPL, EPI, true>(lin.scales_type, a, blocks, s);
+    } else if (lin.bits == 4) {
+        launch_thin_st<4, NPL, EPI, false>(lin.scales_type, a, blocks, s);
+    } else {
+        launch_thin_st<8, NPL, EPI, false>(lin.scales_type, a, blocks, s);
+    }
     return launch_status();
 }
 
 int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, void *out, int out_dtype,
                  int32_t *topk_ids, float *topk_weights, const float *logit_bias, void *ws, size_t ws_bytes,
-                 int flags, int stage_mask, void *stream) {
+                 int flags, int stage_mask, void *stream, bool whole_bias = false) {
     if (x_dtype != SWQ_F32 && x_dtype != SWQ_BF16) return SWQ_ERR_UNSUPPORTED_DTYPE;
     if (stage_mask <= 0 || stage_mask > SWQ_PREFILL_ALL) return SWQ_ERR_INVALID_ARGUMENT;
     int st = check_prefill_layer(layer, T);
@@ -1939,6 +1946,7 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16x = x_dtype == SWQ_BF16;
     const bool thin = thin_tiles(layer, T);
+    if (whole_bias && (!bf16x || !thin)) return SWQ_ERR_LIMIT;  // a decode batch has bf16 x and at most 16 tokens
 
     // x planes for gate/up (nibble_order for 4-bit codes, hi/lo for fp32 x)
     // and the group sums of x: written by the router GEMM as it stages x
@@ -1974,7 +1982,9 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         const bool wide = T >= kRouterWide;
         const int tile = wide ? 2 * kRouterRows : kRouterRows;
         const int blocks = gemm_blocks((T + tile - 1) / tile, g.nblk);
-        if (!wide)
+        if (whole_bias)
+            st = launch_gemm<kSrcBF16, 1, kEpiRows, kSumStage, true>(layer->router, g, blocks, s);
+        else if (!wide)
             st = bf16x ? launch_gemm<kSrcBF16, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s)
                        : launch_gemm<kSrcF32, 1, kEpiRows, kSumStage>(layer->router, g, blocks, s);
         else
@@ -2056,8 +2066,8 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.nblk = (wl.Ih + g.col_block - 1) / g.col_block;
         g.max_tiles = wl.max_tiles;
         if (thin) {
-            st = bf16x ? launch_thin<1, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, s)
-                       : launch_thin<2, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, s);
+            st = bf16x ? launch_thin<1, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, whole_bias, s)
+                       : launch_thin<2, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, false, s);
         } else {
             const int blocks = gemm_blocks(wl.max_tiles, g.nblk);
             st = bf16x ? launch_dma<1, kEpiSwiGLU>(layer->gate, g, blocks, s)
@@ -2090,7 +2100,7 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.col_op = 16;
         g.nblk = (H + g.col_block - 1) / g.col_block;
         g.max_tiles = wl.max_tiles;
-        if (thin) st = launch_thin<2, kEpiRows>(layer->down, g, wl.max_tiles, H, s);
+        if (thin) st = launch_thin<2, kEpiRows>(layer->down, g, wl.max_tiles, H, whole_bias, s);
         else st = launch_dma<2, kEpiRows>(layer->down, g, gemm_blocks(wl.max_tiles, g.nblk), s);
         if (st != SWQ_OK) return st;
     }
@@ -2124,7 +2134,7 @@ size_t grouped_ws_bytes(const swq_moe_layer *l, int batch) {
 int grouped_decode(const swq_moe_layer *layer, const void *x, int x_dtype, int batch, void *out, int out_dtype,
                    int32_t *topk_ids, float *topk_weights, void *ws, size_t ws_bytes, int flags, hipStream_t stream) {
     return prefill_impl(layer, x, x_dtype, batch, out, out_dtype, topk_ids, topk_weights, nullptr, ws, ws_bytes, flags,
-                        SWQ_PREFILL_ALL, stream);
+                        SWQ_PREFILL_ALL, stream, true);
 }
 
 }  // namespace swq
