@@ -815,18 +815,27 @@ __device__ __forceinline__ void ring_wait() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
+// ring_wait<BASE + n>() for n of 0 to 2 (wave-uniform): one branch per count, each with its immediate.
+template <int BASE>
+__device__ __forceinline__ void ring_wait_plus(int n) {
+    if (n <= 0) ring_wait<BASE>();
+    else if (n == 1) ring_wait<BASE + 1>();
+    else ring_wait<BASE + 2>();
+}
+
 // The grouped quantised GEMM of pf_gemm (same tile, lanes and arithmetic) fed
 // by LDS rings: per group, each wave's DMA brings in its share of the 64
-// activation rows (NPL bf16 planes, already in the order the codes need) one
-// group ahead of its use and its 2 x 16 code rows (f32 scales: and their
-// scales) two groups ahead.  2-byte scales come
+// activation rows (NPL bf16 planes, already in the order the codes need) DA - 1
+// groups ahead of its use and its 2 x 16 code rows (f32 scales: and their
+// scales) DA groups ahead.  2-byte scales come
 // from registers: the bias term's scale preload holds every group's, handed
 // between lanes per group.  Activation rows are 128 B; row r
 // keeps its 16 B chunk c in slot c ^ (r & 7) so the matrix-core reads of 16
 // rows at one chunk hit distinct banks.
-template <int BITS, int ST, int NPL, int EPI, int WAVES>
+template <int BITS, int ST, int NPL, int EPI, int DA, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void pf_gemm_dma(const GemmArgs a) {
-    constexpr int DA = 2, DB = 3;                    // groups in the rings of activations and codes
+    static_assert(DA == 2 || (DA == 3 && NPL * (8 / WAVES) <= 2), "ring depths, wait counts");
+    constexpr int DB = DA + 1;                       // groups in the ring of codes (DA: of activations)
     static_assert(WAVES == 4 || WAVES == 8, "waves per workgroup");
     constexpr int MT = 4, ROWS = 64;
     constexpr int AW = 8 / WAVES;                    // 8-row slabs each wave brings in per plane
@@ -1019,22 +1028,29 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
     }
 
-    // ---- the rings: activation rows (mostly L2 hits) one group ahead, codes
-    // two.  Before the loop: B groups 0 and 1, then A group 0.  At group g: wait
-    // until A(g) has landed (B(g) is older), then refill the slots group g-1 used
-    // with A(g+1) and B(g+2) (past NG: group NG-1 again, never read), then
-    // compute g.  Loads return in order, and those issued after A(g) are B(g+1)'s
-    // LB, so at most LB in flight means that A(g) and everything before it have
-    // landed (without a live slab too: B(g) is older than B(g+1)).
+    // ---- the rings: activation rows (mostly L2 hits) DA-1 groups ahead, codes
+    // DB-1.  Before the loop: B groups 0..DB-2, then A groups 0..DA-2.  At group
+    // g: wait until A(g) has landed (B(g) is older), then refill the slots group
+    // g-1 used with A(g+DA-1) and B(g+DB-1) (past NG: group NG-1 again, never
+    // read), then compute g.  Loads return in order, so at most as many in flight
+    // as were issued after A(g) means that it and everything before it have
+    // landed: with DA = 2 B(g+1)'s LB, with DA = 3 the last two steps' LB and the
+    // wave's n = NPL * live copies of the last (group 1, whose A was issued before
+    // the loop: n + LB).  Without a live slab these count the loads after B(g).
 #pragma unroll
     for (int s = 0; s < DB - 1; ++s) issue_b(s, min(s, NG - 1));
-    issue_a(0, 0);
+#pragma unroll
+    for (int s = 0; s < DA - 1; ++s) issue_a(s, min(s, NG - 1));
+    const int nl = NPL * live;
     auto step = [&](int g, int sa, int sb) {
-        issue_a(sa ^ 1, min(g + 1, NG - 1));
+        issue_a(DA == 2 ? sa ^ 1 : sa == 0 ? DA - 1 : sa - 1, min(g + DA - 1, NG - 1));
         issue_b(sb == 0 ? DB - 1 : sb - 1, min(g + DB - 1, NG - 1));
         compute(sa, sb, g);
     };
-    if (0 < NG) ring_wait<0>();
+    if (0 < NG) {
+        if constexpr (DA == 2) ring_wait<0>();
+        else ring_wait_plus<0>(nl);
+    }
     // The scale words were loaded before every ring load, so the wait above
     // has landed them; the compiler cannot know that (it does not count the
     // DMA loads) and would wait for them at their first use in the loop, on
@@ -1049,13 +1065,19 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(bi.s[j][i]));
     if (0 < NG) step(0, 0, 0);
+    if constexpr (DA == 3)
+        if (1 < NG) {
+            ring_wait_plus<LB>(nl);
+            step(1, 1, 1);
+        }
     {
-        int sa = 1, sb = 1;
+        int sa = DA - 1, sb = DA - 1;
 #pragma unroll 1
-        for (int g = 1; g < NG; ++g) {
-            ring_wait<LB>();
+        for (int g = DA - 1; g < NG; ++g) {
+            if constexpr (DA == 2) ring_wait<LB>();
+            else ring_wait_plus<2 * LB>(nl);
             step(g, sa, sb);
-            sa ^= 1;
+            sa = DA == 2 ? sa ^ 1 : sa + 1 == DA ? 0 : sa + 1;
             sb = sb + 1 == DB ? 0 : sb + 1;
         }
     }
@@ -1857,19 +1879,22 @@ int launch_gemm(const swq_qlinear &lin, const GemmArgs &a, int blocks, hipStream
 // 100.8/96.7 where some are busier, 105.0/104.3 at a Zipf load; 4,096 tokens
 // 314.7/301.0 and 310.3/303.9.  Without the branch per wait count, which deeper
 // rings needed, 100.0, 95.4, 103.2, 297 and 298).  Five, with the group sums read
-// at the end instead of held in LDS, spill.
+// at the end instead of held in LDS, spill.  f32 scales, which ride the ring, keep
+// three groups in 4-bit gate/up with bf16 x (256 experts of 512 at 512 tokens 162.9
+// us with two, 152.8 with three; 128 of 768 at 100 tokens 118.7 / 101.9).
 int dma_waves(int bits, int npl) { return (bits == 8 && npl == 2) || (bits == 4 && npl == 1) ? 4 : 8; }
 
 template <int BITS, int NPL, int EPI>
 void launch_dma_st(int stype, const GemmArgs &a, int blocks, hipStream_t s) {
     constexpr int W = (BITS == 8 && NPL == 2) || (BITS == 4 && NPL == 1) ? 4 : 8;
+    constexpr int DA32 = BITS == 4 && NPL == 1 ? 3 : 2;
     const dim3 th(64 * W);
     if (stype == SWQ_F16)
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F16, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F16, NPL, EPI, 2, W>), dim3(blocks), th, 0, s, a);
     else if (stype == SWQ_BF16)
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_BF16, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_BF16, NPL, EPI, 2, W>), dim3(blocks), th, 0, s, a);
     else
-        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F32, NPL, EPI, W>), dim3(blocks), th, 0, s, a);
+        hipLaunchKernelGGL((pf_gemm_dma<BITS, SWQ_F32, NPL, EPI, DA32, W>), dim3(blocks), th, 0, s, a);
 }
 
 template <int NPL, int EPI>

@@ -282,12 +282,13 @@ def test_prefill_router_scales_two_bytes_past_a_word():
 @pytest.mark.parametrize("H,I,Is,bits,x_dtype,f32_scales", [
     (2048, 512, 512, 4, "bf16", False), (384, 384, 128, 4, "bf16", False), (128, 640, 256, 4, "f32", False),
     (640, 128, 384, 8, "bf16", False), (256, 896, 0, 8, "f32", False), (384, 256, 128, 4, "bf16", True),
-    (256, 384, 128, 8, "f32", True)])
+    (256, 384, 128, 8, "f32", True), (128, 128, 128, 4, "bf16", True), (2048, 256, 128, 4, "bf16", True)])
 def test_few_tokens_equal_many(H, I, Is, bits, x_dtype, f32_scales):
     """The GEMM over 16-row tiles (up to six tokens per expert on average: 90 tokens of 60 experts,
     top 4) gives the bits of the one over 64-row tiles: the rows of calls of 1, 8, 9, 16, 17 and 90
     tokens equal those of a call of 91.  Group counts that fill its stages and ones that do not
-    (6, 10, 14 groups), both activation forms, 2- and 4-byte scales."""
+    (6, 10, 14 groups), both activation forms, 2- and 4-byte scales; 4-byte ones with 2, 6 and 32
+    groups under the 64-row kernel's deeper ring."""
     import torch
     shape = synth.MoEShape("few", H, 60, 4, I, Is, expert_bits=bits, router_bits=8, group=64, norm_topk_prob=True)
     gpu = moe.synth_layer(shape, 4000 + H + I, 0)
