@@ -1713,9 +1713,22 @@ int router_kslices(int H) { return (H / kGroupK + kBlockG - 1) / kBlockG; }
 // (f32 x at 256 tokens, 4-bit: 165/170.)  The rule has no code width: with 8-bit codes and bf16 x
 // gate/up alone is slower in 16-row tiles at 16 tokens (56.4/58.8; at 77 109.5/103.7), down's gain
 // is the larger one (39.9/30.5, 80.0/61.0).
+//   Where down's rows fit one stage of the ring (1,024 bits) its tiles only pay the ring's start,
+// and with many pairs that outweighs what gate/up gains: with f32 x, or rows of half a stage, up to
+// kThinShortPairs pairs.  4-bit, 64-row/16-row tiles:
+//   pairs                                  1,024    1,536    2,048    2,560    3,072    4,096
+//   512 experts of 128, top-8, f32 x     121/117  129/128  132/135  140/148  148/151
+//     bf16 x                             112/111  122/122  128/130  134/138  137/142
+//   1,024 of 256, top-16, f32 x          232/226           297/297           330/331  343/354
+//     bf16 x (stays)                     231/210           287/265           322/299  337/317
 constexpr int kThinAvgRows = 6;
-int most_thin_tokens(const swq_moe_layer *l) { return std::max(kThinRows, kThinAvgRows * l->num_experts / l->top_k); }
-bool thin_tiles(const swq_moe_layer *l, int T) { return T <= most_thin_tokens(l); }
+constexpr int kThinShortPairs = 1536;
+int most_thin_tokens(const swq_moe_layer *l, bool bf16x) {
+    int pairs = kThinAvgRows * l->num_experts;
+    if (static_cast<int64_t>(l->moe_intermediate) * l->down.bits <= (bf16x ? 512 : 1024)) pairs = std::min(pairs, kThinShortPairs);
+    return std::max(kThinRows, pairs / l->top_k);
+}
+bool thin_tiles(const swq_moe_layer *l, int T, bool bf16x) { return T <= most_thin_tokens(l, bf16x); }
 
 // Most tiles of up to `cap` rows that T tokens can make.
 int most_tiles(const swq_moe_layer *l, int T, int cap) {
@@ -1733,7 +1746,7 @@ constexpr int kRouterWide = 1024;
 
 struct PfLayout {
     size_t header, counts, logits, sg, ids, wts, pos, tok, tiles, xs_x, xs_h, xa0, xa1, h_hi, h_lo, y, total;
-    int max_tiles, Ih, xs_ld_x, xs_ld_h, kslices;
+    int Ih, xs_ld_x, xs_ld_h, kslices;
 };
 
 PfLayout pf_layout(const swq_moe_layer *l, int T) {
@@ -1747,9 +1760,8 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
     const size_t P = static_cast<size_t>(T) * l->top_k;
     const size_t rows = P + (l->has_shared ? T : 0);
     // the table has room for what any T' <= T needs, in either tile size, so that a workspace
-    // made for T tokens serves fewer too
-    const int thin = most_tiles(l, std::min(T, most_thin_tokens(l)), kThinRows);
-    w.max_tiles = thin_tiles(l, T) ? thin : most_tiles(l, T, kTileRows);
+    // made for T tokens serves fewer too (16-row tiles go furthest with bf16 x)
+    const int tiles = std::max(most_tiles(l, std::min(T, most_thin_tokens(l, true)), kThinRows), most_tiles(l, T, kTileRows));
     w.Ih = std::max(l->moe_intermediate, l->has_shared ? l->shared_intermediate : 0);
     w.header = take(256);  // [1] tile count
     w.counts = P > kGroupSplitPairs ? take(static_cast<size_t>(kGroupSplit) * l->num_experts * 4) : 0;
@@ -1760,7 +1772,7 @@ PfLayout pf_layout(const swq_moe_layer *l, int T) {
     w.wts = take(P * 4);
     w.pos = take(P * 4);
     w.tok = take(rows * 4);
-    w.tiles = take(static_cast<size_t>(std::max(thin, w.max_tiles)) * sizeof(Tile));
+    w.tiles = take(static_cast<size_t>(tiles) * sizeof(Tile));
     w.xs_ld_x = ((l->hidden / kGroupK) + 31) & ~31;  // whole 32-group blocks (the bias MFMA's k)
     w.xs_ld_h = ((w.Ih / kGroupK) + 31) & ~31;
     w.xs_x = take(static_cast<size_t>(T) * w.xs_ld_x * 4);
@@ -1970,7 +1982,8 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
     float *xs_h = reinterpret_cast<float *>(wsb + wl.xs_h);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16x = x_dtype == SWQ_BF16;
-    const bool thin = thin_tiles(layer, T);
+    const bool thin = thin_tiles(layer, T, bf16x);
+    const int max_tiles = most_tiles(layer, T, thin ? kThinRows : kTileRows);
     if (whole_bias && (!bf16x || !thin)) return SWQ_ERR_LIMIT;  // a decode batch has bf16 x and at most 16 tokens
 
     // x planes for gate/up (nibble_order for 4-bit codes, hi/lo for fp32 x)
@@ -2089,12 +2102,12 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.col_block = 16 * dma_waves(layer->gate.bits, bf16x ? 1 : 2);
         g.col_op = 0;
         g.nblk = (wl.Ih + g.col_block - 1) / g.col_block;
-        g.max_tiles = wl.max_tiles;
+        g.max_tiles = max_tiles;
         if (thin) {
-            st = bf16x ? launch_thin<1, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, whole_bias, s)
-                       : launch_thin<2, kEpiSwiGLU>(layer->gate, g, wl.max_tiles, wl.Ih, false, s);
+            st = bf16x ? launch_thin<1, kEpiSwiGLU>(layer->gate, g, max_tiles, wl.Ih, whole_bias, s)
+                       : launch_thin<2, kEpiSwiGLU>(layer->gate, g, max_tiles, wl.Ih, false, s);
         } else {
-            const int blocks = gemm_blocks(wl.max_tiles, g.nblk);
+            const int blocks = gemm_blocks(max_tiles, g.nblk);
             st = bf16x ? launch_dma<1, kEpiSwiGLU>(layer->gate, g, blocks, s)
                        : launch_dma<2, kEpiSwiGLU>(layer->gate, g, blocks, s);
         }
@@ -2124,9 +2137,9 @@ int prefill_impl(const swq_moe_layer *layer, const void *x, int x_dtype, int T, 
         g.col_block = 32 * dma_waves(layer->down.bits, 2);
         g.col_op = 16;
         g.nblk = (H + g.col_block - 1) / g.col_block;
-        g.max_tiles = wl.max_tiles;
-        if (thin) st = launch_thin<2, kEpiRows>(layer->down, g, wl.max_tiles, H, whole_bias, s);
-        else st = launch_dma<2, kEpiRows>(layer->down, g, gemm_blocks(wl.max_tiles, g.nblk), s);
+        g.max_tiles = max_tiles;
+        if (thin) st = launch_thin<2, kEpiRows>(layer->down, g, max_tiles, H, whole_bias, s);
+        else st = launch_dma<2, kEpiRows>(layer->down, g, gemm_blocks(max_tiles, g.nblk), s);
         if (st != SWQ_OK) return st;
     }
     // 5. weighted combine in pick order, then the gated shared expert

@@ -207,7 +207,7 @@ def test_prefill_workspace_query(lib):
     assert lib.swq_moe_prefill_workspace_bytes(ctypes.byref(layer(router=lin(256, 2048, 8, group=32))), 8) == 0
 
 
-@pytest.mark.parametrize("E,K,H,I", [(1023, 1, 128, 128), (721, 1, 128, 128), (1024, 4, 128, 128), (8, 2, 128, 128),
+@pytest.mark.parametrize("E,K,H,I", [(1023, 1, 128, 128), (721, 1, 128, 128), (1024, 4, 128, 128), (8, 2, 128, 128), (1024, 1, 128, 256), (900, 1, 256, 256),
                                      (1, 1, 128, 128), (256, 8, 2048, 512), (512, 10, 2048, 512)])
 def test_prefill_workspace_serves_fewer_tokens(lib, E, K, H, I):
     """The bytes never fall as the tokens grow, also where the tiles change from 16 rows to 64 (6 E / K

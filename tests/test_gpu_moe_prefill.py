@@ -305,6 +305,26 @@ def test_few_tokens_equal_many(H, I, Is, bits, x_dtype, f32_scales):
         assert torch.equal(ids, want_ids[:T]) and torch.equal(w, want_w[:T]) and torch.equal(out, want[:T]), T
 
 
+@pytest.mark.parametrize("I,x_dtype", [(128, "bf16"), (128, "f32"), (256, "f32"), (256, "bf16")])
+def test_short_down_rows_equal_on_either_side(I, x_dtype):
+    """Where down's rows fit one stage of the 16-row kernel's ring the tiles change size at 1,536 pairs
+    already (but for 256 inputs with bf16 x, at six rows per expert): 192 tokens of top 8 have those
+    tiles, 193 the 64-row ones, 390 and 391 stand on the other line, and every row has the same bits."""
+    import torch
+    shape = synth.MoEShape("short", 256, 520, 8, I, 128, expert_bits=4, router_bits=8, group=64, norm_topk_prob=True)
+    gpu = moe.synth_layer(shape, 4400 + I, 0)
+    x, _ = _x(78 + I, 391, 256)
+    if x_dtype == "f32":
+        x = x.float() * 1.1
+    print(f"short down rows: I {I} x {x_dtype}", flush=True)
+    ws = gpu.new_prefill_workspace(391)
+    want, want_ids, want_w = gpu.prefill(x, ws=ws)
+    for T in (191, 192, 193, 390):
+        out, ids, w = gpu.prefill(x[:T].contiguous(), ws=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want_ids[:T]) and torch.equal(w, want_w[:T]) and torch.equal(out, want[:T]), T
+
+
 @pytest.mark.parametrize("E,K,T,x_dtype", [(60, 9, 911, "bf16"), (256, 8, 1024, "f32"), (256, 8, 1025, "bf16"),
                                            (513, 5, 2049, "bf16"), (256, 8, 3073, "bf16"), (520, 16, 1311, "f32")])
 def test_many_tokens_equal_few(E, K, T, x_dtype):
