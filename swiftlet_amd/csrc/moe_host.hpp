@@ -170,8 +170,8 @@ inline size_t grouped_ws_base(const FusedLayout &f) { return align256(f.total); 
 // grouped:
 //   batch                          5      6      7      8      11      16
 //   256 experts top-8 (3.1 M
-//   codes a pair)                58/55  65/55  72/58  78/59  103/68  135/79
-//   512 experts top-10           71/61  79/63  89/67  95/71  126/84  170/98
+//   codes a pair)                57/53  65/55  72/58  79/59  103/69  137/82
+//   512 experts top-10           71/62  79/63  89/67  98/73  126/85  172/99
 // Its bias term takes b - 16 s in 24 significant bits, which hold all that f16 and
 // bf16 scales can make of it (exponents up to 13 apart) but not f32 ones.  f32
 // scales on any matrix, f32 activations and 8-bit experts stay with the three
